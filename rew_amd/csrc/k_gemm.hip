@@ -1203,6 +1203,8 @@ bool gemm_epilogue_ok(const GemmArgs& g) {
 
 const char* gemm_variant(const GemmArgs& g) {
   bool akc, bkc;
+  if (gemm_strip_better(&g, 1))
+    return g.epi == EPI_SWIGLU ? "gemm_lds_swiglu_strip" : "gemm_lds_nn_strip";
   if (use_lds(g)) {
     gemm_lds_ok(g, &bkc);
     return g.epi == EPI_SWIGLU ? "gemm_lds_swiglu" : (bkc ? "gemm_lds_tn" : "gemm_lds_nn");
@@ -1220,6 +1222,10 @@ const char* gemm_variant(const GemmArgs& g) {
 void launch_gemm(const GemmArgs& g, hipStream_t stream) {
   if (g.M == 0 || g.N == 0 || g.batch == 0) return;
   bool akc, bkc;
+  if (gemm_strip_better(&g, 1)) {
+    launch_gemm_strip(&g, 1, stream);
+    return;
+  }
   if (use_lds(g)) {
     launch_gemm_lds(g, nullptr, stream);
     return;

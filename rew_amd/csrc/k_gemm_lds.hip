@@ -1044,6 +1044,10 @@ bool gemm_multi_ok(const GemmArgs* segs, int n) {
 
 void launch_gemm_multi(const GemmArgs* segs, int n, hipStream_t stream) {
   if (!gemm_multi_ok(segs, n)) fail(REW_MI355X_ERR_INVALID, "internal: GEMM set not launchable");
+  if (gemm_strip_better(segs, n)) {
+    launch_gemm_strip(segs, n, stream);
+    return;
+  }
   GemmSegs gs;
   std::memset(&gs, 0, sizeof gs);
   gs.n = n;

@@ -168,6 +168,11 @@ struct GemmSegs {
 };
 bool gemm_multi_ok(const GemmArgs* segs, int n);
 void launch_gemm_multi(const GemmArgs* segs, int n, hipStream_t stream);
+// The strip kernel (k_gemm_strip.hip) for bf16 products of few rows or few
+// tiles; `better` also says whether it takes the set (same conditions as
+// gemm_multi_ok, N-contiguous B) in place of the 256x256 kernels.
+bool gemm_strip_better(const GemmArgs* segs, int n);
+void launch_gemm_strip(const GemmArgs* segs, int n, hipStream_t stream);
 // Whether launch_gemm runs g with its epilogue (EPI_SWIGLU needs the large
 // dual kernel; the others run on every MFMA kernel).
 bool gemm_epilogue_ok(const GemmArgs& g);

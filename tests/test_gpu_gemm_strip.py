@@ -1,0 +1,105 @@
+"""GPU parity of the strip GEMM (k_gemm_strip.hip) at the edges of its tiles,
+its partial last k-tile and its split sums, against an fp64 product.
+
+Bound per element: the product, its sum with the bias and that with the
+residual are each rounded to bf16 once (at most 2^-8 of the value rounded, so
+3 * 2^-8 of the magnitudes), and the fp32 sums add K * 2^-24 of the absolute
+products.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from rew_amd import eager as E
+from rew_amd import nn
+from rew_amd import ops as O
+from rew_amd.eager import DType
+
+
+def _bf16(r, shape, scale):
+    return E.bf16_bits_to_f32(E.f32_to_bf16_bits((r.standard_normal(shape) * scale)
+                                                 .astype(np.float32))).reshape(shape)
+
+
+def _dev(a):
+    return E.fromHost(a, DType.BFLOAT16)
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (1, 64, 8),          # one row, one k-tile, fewer columns than a wave
+    (32, 8, 128),        # K below a k-tile; exactly one tile
+    (33, 136, 264),      # a second row block, K and N remainders
+    (64, 1000, 392),     # partial last k-tile with 16 of them
+    (160, 192, 1032),    # five row blocks
+    (161, 2048, 520),    # split sums with a ragged second row tile
+    (8, 14336, 256),     # the deepest split
+    (129, 1032, 136),    # split, partial last k-tile in the last split only
+])
+def test_strip_linear_and_residual(gpu, M, K, N):
+    r = np.random.default_rng(M * 7 + K + N)
+    x, w, b = _bf16(r, (M, K), 1.0), _bf16(r, (K, N), 0.05), _bf16(r, (N,), 1.0)
+    res = _bf16(r, (M, N), 1.0)
+    xt, wt, bt, rt = _dev(x), _dev(w), _dev(b), _dev(res)
+    exact = x.astype(np.float64) @ w.astype(np.float64)
+    mag = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64)
+    for add in (False, True):
+        def fn():
+            y = nn.Linear(wt, bt).forward(xt)
+            return O.add(rt, y) if add else y
+        E.profileBegin()
+        got = E.toHostF32(fn())
+        names = [n for n, _, _ in E.profileEnd()]
+        assert len(names) == 1 and names[0].startswith("gemm_lds_nn_strip+bias"), names
+        want = exact + b + (res if add else 0)
+        size = np.abs(exact) + np.abs(b) + (np.abs(res) if add else 0)
+        assert np.all(np.abs(got - want) <= 3 * 2.0 ** -8 * size + K * 2.0 ** -24 * mag)
+        for _ in range(3):  # the split sums run in one order whatever finishes last
+            np.testing.assert_array_equal(E.toHostF32(fn()), got)
+
+
+@pytest.mark.parametrize("T,H,I", [(1, 64, 8), (33, 136, 264), (40, 2048, 384), (150, 1032, 200)])
+def test_strip_swiglu(gpu, oracle, T, H, I):
+    r = np.random.default_rng(T + H + I)
+    x = _bf16(r, (T, H), 1.0)
+    ws = [_bf16(r, s, 0.05) for s in ((H, I), (H, I), (I, H))]
+    bs = [_bf16(r, (n,), 0.5) for n in (I, I, H)]
+    ffn = nn.GatedFeedForward(*[nn.Linear(_dev(w), _dev(b)) for w, b in zip(ws, bs)])
+    E.profileBegin()
+    got = E.toHostF32(ffn.forward(_dev(x.reshape(1, T, H)))).reshape(T, H)
+    names = [n for n, _, _ in E.profileEnd()]
+    assert any(n.startswith("gemm_lds_swiglu_strip") for n in names), names
+    want = oracle.gated_ffn(x, ws[0], bs[0], ws[1], bs[1], ws[2], bs[2], True)
+    # the oracle rounds where the op sequence does; sums in another order move
+    # a rounding of the hidden row by one bf16 ulp now and then
+    assert np.linalg.norm(got - want) <= 2e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("B,S", [(1, 1), (2, 33)])
+def test_strip_projections_with_rope(gpu, oracle, B, S):
+    """The q / k / v projections of a few tokens in one launch, k split."""
+    H, nh, nkv, hd = 1024, 8, 2, 128
+    r = np.random.default_rng(B + S)
+    x = _bf16(r, (B * S, H), 1.0)
+    lin = [(_bf16(r, (H, n), 0.03), _bf16(r, (n,), 0.2)) for n in (nh * hd, nkv * hd, nkv * hd)]
+    rope = nn.RotaryPositionEncoding.init(hd, S, 10000.0)
+    c, s = nn.rope_tables(hd, S, 10000.0)
+
+    def fn():
+        xt = _dev(x)
+        outs = []
+        for (w, b), n, rot in zip(lin, (nh, nkv, nkv), (True, True, False)):
+            y = O.reshape(nn.Linear(_dev(w), _dev(b)).forward(xt), [B, S, n, hd])
+            y = O.transpose(y, [0, 2, 1, 3])
+            outs.append(rope.forward(y) if rot else O.add(y, y))
+        return outs
+
+    E.profileBegin()
+    outs = [E.toHostF32(t) for t in fn()]
+    names = [n for n, _, _ in E.profileEnd()]
+    assert any(n.startswith("gemm_lds_nn{") and n.count("+rope") == 2 for n in names), names
+    for got, (w, b), n, rot in zip(outs, lin, (nh, nkv, nkv), (True, True, False)):
+        y = oracle.round_bf16(oracle.round_bf16((x.astype(np.float64) @ w).astype(np.float32)) + b)
+        y = y.reshape(B, S, n, hd).transpose(0, 2, 1, 3)
+        want = oracle.rope(np.ascontiguousarray(y), c, s, offset=0) if rot else y + y
+        assert np.linalg.norm(got - want) <= 4e-3 * np.linalg.norm(want)
