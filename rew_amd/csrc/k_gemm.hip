@@ -1114,9 +1114,279 @@ static bool f32_narrow_ok(const GemmArgs& g) {
          g.M / 16 < (1 << 30);
 }
 
-// Problems whose 64x64 tiles would leave most CUs idle run 16x16 tiles.
+// ---------------------------------------------------------------------------
+// f32 on the matrix cores
+// ---------------------------------------------------------------------------
+//
+// v_mfma_f32_16x16x1_4b: one k-step of four 16 x 16 blocks, each output
+// rounded as fmaf(a, b, acc), so a chain of them over k gives the bits of
+// gemm_generic_kernel's fmaf chain at the matrix cores' 256 FLOP per clock
+// and CU (the generic kernel's scalar loads and LDS reads kept it at 13-30
+// TFLOP/s: 2000 x 1024 x 2816 433 -> 146 us, 8192 x 2048 x 2048 2656 -> 658 us
+// or 104 TFLOP/s, 64 of 500 x 64 x 500 108 -> 40 us).  A tile of 64 RW rows x 64 columns per workgroup, each wave RW
+// times 16 rows x 64 columns (the A rows repeated in all four blocks), so a
+// wave runs RW chains; k-tiles of 32 through two LDS buffers, the next one in
+// registers while the current one is multiplied.  The operands of four
+// k-steps are read one group ahead, over the barrier too: a chain waits
+// between its MFMAs for whatever is not there yet, and with one or two waves
+// per SIMD nothing else covers it.
+//
+// AM / BM say how an operand is read: VEC_K 16-byte loads along k, VEC_N
+// (B) 16-byte loads along n, ANY 4-byte loads at any strides, lanes along
+// the contiguous one.
+enum { VEC_K = 0, VEC_N = 1, ANY = 2 };
+constexpr int kFT = 64, kFK = 32;  // tile columns (rows: RW times), k-tile
+constexpr int kFG = 8;             // k-steps per group of LDS reads
+// From this many 128-row tiles (four per CU) the 32 x 32 blocks are faster:
+// 8192 x 2048 x 2048 658 us against 710, 1000 x 1000 x 3000 (376 tiles) 91
+// against 82.
+constexpr int64_t kF32TwoTiles = 1024;
+
+template <int RW, int AM, int BM>
+__global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t tiles_m,
+                                                            int64_t tiles_n) {
+  constexpr int FM = kFT * RW;
+  constexpr int KP = kFK + 4;  // k-major rows: 16-byte reads of 16 rows on distinct banks
+  constexpr int NP = kFT + 4;
+  constexpr bool BK_ROWS = BM == VEC_K;  // B in LDS as [n][k], else [k][n]
+  __shared__ __attribute__((aligned(16))) float As[2][FM][KP];
+  __shared__ __attribute__((aligned(16))) float Bs[2][BK_ROWS ? kFT * KP : kFK * NP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+
+  // XCD-contiguous ranges, then groups of 8 row tiles walked down the columns
+  int64_t t = blockIdx.x, b;
+  {
+    const int64_t total = tiles_m * tiles_n * g.batch, q = total / 8, rr = total % 8, x = t % 8;
+    t = x * q + (x < rr ? x : rr) + t / 8;
+    b = t / (tiles_m * tiles_n);
+    t -= b * tiles_m * tiles_n;
+  }
+  const int64_t grp = t / (8 * tiles_n), first = grp * 8;
+  const int64_t gsz = min((int64_t)8, tiles_m - first), r8 = t - grp * 8 * tiles_n;
+  const int m0 = (int)(first + r8 % gsz) * FM, n0 = (int)(r8 / gsz) * kFT;
+  const float* A = (const float*)g.a + b * g.a_sb;
+  const float* B = (const float*)g.b + b * g.b_sb;
+
+  // two sets of registers, each loaded two k-tiles ahead (a tile is 0.5 us of
+  // MFMAs for one wave, a load from HBM more)
+  float rga[2][8 * RW], rgb[2][8];
+  // element (row, k) of the tile for this thread's slot i (ANY)
+  const bool a_k = g.a_sk == 1 || g.a_sm != 1, b_k = g.b_sk == 1 && g.b_sn != 1;
+  auto put4 = [](float* d, const float4& v) {
+    d[0] = v.x;
+    d[1] = v.y;
+    d[2] = v.z;
+    d[3] = v.w;
+  };
+  auto fetch = [&](int k0, int set) {
+    float* ra = rga[set];
+    float* rb = rgb[set];
+#pragma unroll
+    for (int i = 0; i < (AM == VEC_K ? 2 : 8) * RW; ++i) {
+      const int e = tid + i * 256;
+      if constexpr (AM == VEC_K) {
+        const int row = min(m0 + (e >> 3), M - 1), k = k0 + (e & 7) * 4;
+        put4(ra + 4 * i, *(const float4*)(A + row * g.a_sm + min(k, K - 4)));
+      } else {
+        const int row = min(m0 + (a_k ? e >> 5 : e % FM), M - 1);
+        const int k = k0 + (a_k ? e & 31 : e / FM);
+        ra[i] = A[row * g.a_sm + min(k, K - 1) * g.a_sk];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < (BM == ANY ? 8 : 2); ++i) {
+      const int e = tid + i * 256;
+      if constexpr (BM == VEC_K) {
+        const int col = min(n0 + (e >> 3), N - 1), k = k0 + (e & 7) * 4;
+        put4(rb + 4 * i, *(const float4*)(B + col * g.b_sn + min(k, K - 4)));
+      } else if constexpr (BM == VEC_N) {
+        const int k = k0 + (e >> 4), n = min(n0 + (e & 15) * 4, N - 4);
+        put4(rb + 4 * i, *(const float4*)(B + min(k, K - 1) * g.b_sk + n));
+      } else {
+        const int n = min(n0 + (b_k ? e >> 5 : e & 63), N - 1);
+        const int k = k0 + (b_k ? e & 31 : e >> 6);
+        rb[i] = B[min(k, K - 1) * g.b_sk + n * g.b_sn];
+      }
+    }
+  };
+  // the registers of set `set` (k-tile k0) into buffer s, zeros past K by a
+  // mask (a select the compiler turns into a branch around the load, and
+  // then waits for the load on the spot)
+  auto stage = [&](int s, int set, int k0) {
+    const float* ra = rga[set];
+    const float* rb = rgb[set];
+    auto keep = [&](float v, int k) { return vm::as_f(vm::as_u(v) & (uint32_t)((k - K) >> 31)); };
+    auto keep4 = [&](const float* v, int k) {
+      return make_float4(keep(v[0], k), keep(v[1], k), keep(v[2], k), keep(v[3], k));
+    };
+#pragma unroll
+    for (int i = 0; i < (AM == VEC_K ? 2 : 8) * RW; ++i) {
+      const int e = tid + i * 256;
+      if constexpr (AM == VEC_K) {
+        *(float4*)&As[s][e >> 3][(e & 7) * 4] = keep4(ra + 4 * i, k0 + (e & 7) * 4);
+      } else {
+        const int k = a_k ? e & 31 : e / FM;
+        As[s][a_k ? e >> 5 : e % FM][k] = keep(ra[i], k0 + k);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < (BM == ANY ? 8 : 2); ++i) {
+      const int e = tid + i * 256;
+      if constexpr (BM == VEC_K) {
+        *(float4*)&Bs[s][(e >> 3) * KP + (e & 7) * 4] = keep4(rb + 4 * i, k0 + (e & 7) * 4);
+      } else if constexpr (BM == VEC_N) {
+        *(float4*)&Bs[s][(e >> 4) * NP + (e & 15) * 4] = keep4(rb + 4 * i, k0 + (e >> 4));
+      } else {
+        const int k = b_k ? e & 31 : e >> 6;
+        Bs[s][k * NP + (b_k ? e >> 5 : e & 63)] = keep(rb[i], k0 + k);
+      }
+    }
+  };
+
+  // one chain of MFMAs per wave: 16 rows x four blocks of 16 columns (RW 1)
+  // or 32 rows x two blocks of 32 (RW 2)
+  typedef float acc_t __attribute__((ext_vector_type(16 * RW)));
+  constexpr int WR = 16 * RW;
+  acc_t acc;
+#pragma unroll
+  for (int e = 0; e < 16 * RW; ++e) acc[e] = 0.0f;
+  // kFG k-steps of this lane's operands: group q of buffer s
+  float av[2][kFG], bv[2][kFG];
+  auto read = [&](int s, int q, int slot) {
+#pragma unroll
+    for (int x = 0; x < kFG; x += 4) {
+      const float4 v = *(const float4*)&As[s][wave * WR + (lane & (WR - 1))][q * kFG + x];
+      av[slot][x] = v.x; av[slot][x + 1] = v.y; av[slot][x + 2] = v.z; av[slot][x + 3] = v.w;
+    }
+    if constexpr (BK_ROWS) {
+#pragma unroll
+      for (int x = 0; x < kFG; x += 4) {
+        const float4 v = *(const float4*)&Bs[s][lane * KP + q * kFG + x];
+        bv[slot][x] = v.x; bv[slot][x + 1] = v.y; bv[slot][x + 2] = v.z; bv[slot][x + 3] = v.w;
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < kFG; ++x) bv[slot][x] = Bs[s][(q * kFG + x) * NP + lane];
+    }
+  };
+  auto multiply = [&](int slot) {
+#pragma unroll
+    for (int x = 0; x < kFG; ++x) {
+      if constexpr (RW == 1)
+        acc = __builtin_amdgcn_mfma_f32_16x16x1f32(av[slot][x], bv[slot][x], acc, 0, 0, 0);
+      else
+        acc = __builtin_amdgcn_mfma_f32_32x32x1f32(av[slot][x], bv[slot][x], acc, 0, 0, 0);
+    }
+  };
+  constexpr int Q = kFK / kFG;
+  // k-tile k0 from buffer s, whose registers (set s) are free again; the
+  // next one goes from set s ^ 1 to buffer s ^ 1, whose last reader passed
+  // the barrier of the step before.  (Loads past K read the last k: no branch
+  // around them, at which the compiler would wait.)
+  auto step = [&](int k0, int s) {
+    fetch(k0 + 2 * kFK, s);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      if (q < Q - 1) read(s, q + 1, (q + 1) & 1);
+      else read(s ^ 1, 0, 0);  // (past the last k-tile: never used)
+      multiply(q & 1);
+      if (q == Q - 3) stage(s ^ 1, s ^ 1, k0 + kFK);
+      // Spread the rest between the MFMAs: a wave issues in order, and an MFMA
+      // whose chain is not ready holds back what follows it.
+#pragma unroll
+      for (int x = 0; x < kFG; ++x) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
+        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // VALU
+        if (q == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);       // load
+        if (q == Q - 3) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // DS write
+      }
+      if (q == Q - 2) {
+        // (not __syncthreads, which would also wait for the loads in flight)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+      }
+    }
+  };
+  fetch(0, 0);
+  fetch(kFK, 1);
+  stage(0, 0, 0);
+  __syncthreads();
+  read(0, 0, 0);
+  for (int k0 = 0;; k0 += 2 * kFK) {
+    step(k0, 0);
+    if (k0 + kFK >= K) break;
+    step(k0 + kFK, 1);
+    if (k0 + 2 * kFK >= K) break;
+  }
+  // RW 1: register 4 j + r holds row 4 (lane / 16) + r, column 16 j + lane % 16;
+  // RW 2: register 16 j + r row 8 (r / 4) + 4 (lane / 32) + r % 4, column
+  // 32 j + lane % 32
+#pragma unroll
+  for (int e = 0; e < 16 * RW; ++e) {
+    const int row = RW == 1 ? 4 * (lane >> 4) + (e & 3)
+                            : 8 * ((e & 15) >> 2) + 4 * (lane >> 5) + (e & 3);
+    const int col = RW == 1 ? 16 * (e >> 2) + (lane & 15) : 32 * (e >> 4) + (lane & 31);
+    const int m = m0 + wave * WR + row, n = n0 + col;
+    if (m < M && n < N)
+      ((float*)g.c)[b * g.c_sb + m * g.c_sm + n] = epi_value(g, b, m, n, acc[e]);
+  }
+}
+
+// f32 operands and result, and index arithmetic that fits 32 bits.
+static bool f32_mfma_ok(const GemmArgs& g) {
+  constexpr int64_t kLim = (int64_t)1 << 30;
+  return g.dtype == REW_DT_FLOAT32 && g.c_dtype == REW_DT_FLOAT32 && g.K > 0 && g.M < kLim &&
+         g.N < kLim && g.K < kLim &&
+         ((g.M + kFT - 1) / kFT) * ((g.N + kFT - 1) / kFT) * g.batch < kLim &&
+         g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE;
+}
+
+static void launch_gemm_f32_mfma(const GemmArgs& g, hipStream_t stream) {
+  auto vec = [&](const void* p, int64_t sb, int64_t s) {
+    return ((uintptr_t)p & 15) == 0 && sb % 4 == 0 && s % 4 == 0;
+  };
+  int64_t tm = (g.M + 2 * kFT - 1) / (2 * kFT);
+  const int64_t tn = (g.N + kFT - 1) / kFT;
+  const bool two = tm * tn * g.batch >= kF32TwoTiles;
+  if (!two) tm = (g.M + kFT - 1) / kFT;
+  const bool avk = g.a_sk == 1 && g.K % 4 == 0 && vec(g.a, g.a_sb, g.a_sm);
+  const bool bvk = g.b_sk == 1 && g.K % 4 == 0 && vec(g.b, g.b_sb, g.b_sn);
+  const bool bvn = g.b_sn == 1 && g.N % 4 == 0 && vec(g.b, g.b_sb, g.b_sk);
+  const dim3 grid((unsigned)(tm * tn * g.batch));
+#define REW_F32_MFMA(AM, BM)                                                                     \
+  do {                                                                                          \
+    if (two)                                                                                    \
+      hipLaunchKernelGGL((gemm_f32_mfma_kernel<2, AM, BM>), grid, dim3(256), 0, stream, g, tm,  \
+                         tn);                                                                   \
+    else                                                                                        \
+      hipLaunchKernelGGL((gemm_f32_mfma_kernel<1, AM, BM>), grid, dim3(256), 0, stream, g, tm,  \
+                         tn);                                                                   \
+  } while (0)
+  if (avk) {
+    if (bvn) REW_F32_MFMA(VEC_K, VEC_N);
+    else if (bvk) REW_F32_MFMA(VEC_K, VEC_K);
+    else REW_F32_MFMA(VEC_K, ANY);
+  } else {
+    if (bvn) REW_F32_MFMA(ANY, VEC_N);
+    else if (bvk) REW_F32_MFMA(ANY, VEC_K);
+    else REW_F32_MFMA(ANY, ANY);
+  }
+#undef REW_F32_MFMA
+}
+
+// Problems whose 64x64 tiles would leave most CUs idle run 16x16 tiles, until
+// those fill the CUs several times over.  The matrix-core kernel takes about
+// 6 us + 24 ns per k-step whatever its tiles leave idle; the 16x16 tiles are
+// ahead of that up to 32 tiles of 64x64 (128 x 1024 x 1024: 29 us against 31;
+// 333 x 1024 x 512: 46 against 31), or 80 where K is short (333 x 256 x 512:
+// 12 against 14), and no more once K passes the slab they hold in LDS
+// (333 x 2816 x 1024: 178 against 71).
 static bool small_ok(const GemmArgs& g) {
   const int64_t tiles64 = ((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
+  if (f32_mfma_ok(g)) return g.K <= kSmallWholeK && tiles64 <= (g.K >= 512 ? 32 : 80);
   return tiles64 < 128 && g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE;
 }
 
@@ -1211,7 +1481,8 @@ const char* gemm_variant(const GemmArgs& g) {
   }
   if (g.epi == EPI_SWIGLU) return "gemm_bf16_256_swiglu";
   if (!mfma_ok(g, &akc, &bkc))
-    return f32_narrow_ok(g) ? "gemm_f32_narrow" : (small_ok(g) ? "gemm_f32_small" : "gemm_generic");
+    return f32_narrow_ok(g) ? "gemm_f32_narrow" : (small_ok(g) ? "gemm_f32_small"
+                                           : f32_mfma_ok(g) ? "gemm_generic_mfma" : "gemm_generic");
   if (use_256(g, akc)) return bkc ? "gemm_bf16_256_tn" : "gemm_bf16_256_nn";
   if (akc && bkc) return "gemm_bf16_mfma_tn";
   if (akc) return "gemm_bf16_mfma_nn";
@@ -1259,6 +1530,8 @@ void launch_gemm(const GemmArgs& g, hipStream_t stream) {
                        stream, g);
   } else if (small_ok(g)) {
     launch_gemm_small(g, stream);
+  } else if (f32_mfma_ok(g)) {
+    launch_gemm_f32_mfma(g, stream);
   } else {
     dim3 grid((unsigned)((g.N + 63) / 64), (unsigned)((g.M + 63) / 64),
               (unsigned)(g.batch < 65535 ? g.batch : 65535));

@@ -1,0 +1,81 @@
+"""GPU parity of the f32 matrix-core GEMM (gemm_f32_mfma_kernel).  Each output
+is the fmaf chain over k that the 16 x 16 kernel runs, so a slice of a
+product, small enough for that kernel, has the same bits as the product's."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from rew_amd import eager as E
+from rew_amd import nn
+from rew_amd import ops as O
+
+
+def dev(a):
+    return E.fromHost(np.ascontiguousarray(a, np.float32))
+
+
+def run(fn):
+    E.profileBegin()
+    out = E.toHost(fn())
+    return out, [n for n, _, _ in E.profileEnd()]
+
+
+FORMS = {"nn": ((1, 0), lambda a, b: O.matmul(dev(a), dev(b))),
+         "nt": ((1, 1), lambda a, b: O.dotGeneral(dev(a), dev(b.T), [], [], [1], [1])),
+         "tn": ((0, 0), lambda a, b: O.dotGeneral(dev(a.T), dev(b), [], [], [0], [0])),
+         "tt": ((0, 1), lambda a, b: O.dotGeneral(dev(a.T), dev(b.T), [], [], [0], [1]))}
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("M,K,N", [
+    (577, 100, 641),    # remainders of every tile edge; 4-byte loads along m and n
+    (640, 1, 640),      # one k-step
+    (640, 32, 644),     # exactly one k-tile
+    (600, 33, 700),     # one past it, odd K
+    (1100, 96, 8260),   # 128-row tiles (9 x 130 of them)
+])
+def test_chain_equals_small_kernel(gpu, oracle, form, M, K, N):
+    r = np.random.default_rng(M + K + N)
+    a = r.standard_normal((M, K)).astype(np.float32)
+    b = (r.standard_normal((K, N)) * 10.0 ** r.integers(-3, 3, (K, N))).astype(np.float32)
+    a[3, 0], b[0, 5] = np.inf, np.nan
+    _, f = FORMS[form]
+    got, names = run(lambda: f(a, b))
+    assert any(n.startswith("gemm_generic_mfma") for n in names), names
+    for m0, n0 in ((0, 0), (M - 33, N - 65), (M // 2, N // 3)):
+        ref, names = run(lambda: f(a[m0:m0 + 33], b[:, n0:n0 + 65]))
+        assert any(n.startswith("gemm_f32_small") for n in names), names
+        part = got[m0:m0 + 33, n0:n0 + 65]
+        nan = np.isnan(ref)
+        np.testing.assert_array_equal(np.isnan(part), nan)
+        np.testing.assert_array_equal(part[~nan].view(np.uint32), ref[~nan].view(np.uint32))
+    rows = slice(4, 40)  # away from the infinity
+    want = a[rows].astype(np.float64) @ b[:, 6:].astype(np.float64)
+    bound = (K + 1) * 2.0 ** -24 * (np.abs(a[rows]).astype(np.float64) @ np.abs(b[:, 6:]))
+    assert np.all(np.abs(got[rows, 6:] - want) <= bound)
+
+
+def test_batches_and_epilogues(gpu):
+    r = np.random.default_rng(5)
+    B, M, K, N = 6, 333, 65, 331
+    a, b = r.standard_normal((B, M, K)), r.standard_normal((B, K, N))
+    got, names = run(lambda: O.dotGeneral(dev(a), dev(b), [0], [0], [2], [1]))
+    assert any(n.startswith("gemm_generic_mfma") for n in names), names
+    a32, b32 = a.astype(np.float32), b.astype(np.float32)
+    want = np.matmul(a32.astype(np.float64), b32.astype(np.float64))
+    bound = (K + 1) * 2.0 ** -24 * np.matmul(np.abs(a32).astype(np.float64), np.abs(b32))
+    assert np.all(np.abs(got - want) <= bound)
+    x, w, bias, res = a32[0], b32[0], r.standard_normal(N).astype(np.float32), got[1]
+
+    def lin():
+        return nn.Linear(dev(w), dev(bias)).forward(dev(x))
+
+    x = np.repeat(x, 4, 0)
+    res = np.repeat(res, 4, 0)
+    plain, _ = run(lambda: O.matmul(dev(x), dev(w)))
+    for fn, ref in ((lin, plain + bias), (lambda: O.add(dev(res), lin()), res + (plain + bias)),
+                    (lambda: nn.relu(lin()), np.maximum(plain + bias, 0))):
+        out, names = run(fn)
+        assert len(names) == 1 and names[0].startswith("gemm_generic_mfma+bias"), names
+        np.testing.assert_array_equal(out, ref)
