@@ -933,6 +933,7 @@ bool gemm_lds_ok(const GemmArgs& g, bool* b_kc) {
   auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   if (g.dtype != REW_DT_BFLOAT16 || g.c_dtype != REW_DT_BFLOAT16) return false;
   if (g.K <= 0 || g.K % 8 || g.N % 8 || g.M <= 0) return false;
+  if (g.a_sm < 0 || g.b_sk < 0 || g.b_sn < 0) return false;  // (unsigned buffer offsets)
   if (g.a_sk != 1 || g.a_sm % 8 || g.a_sb % 8 || !al16(g.a)) return false;
   if (g.b_sk == 1 && g.b_sn % 8 == 0 && g.b_sb % 8 == 0) *b_kc = true;
   else if (g.b_sn == 1 && g.b_sk % 8 == 0 && g.b_sb % 8 == 0) *b_kc = false;

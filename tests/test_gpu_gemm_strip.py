@@ -103,3 +103,17 @@ def test_strip_projections_with_rope(gpu, oracle, B, S):
         y = y.reshape(B, S, n, hd).transpose(0, 2, 1, 3)
         want = oracle.rope(np.ascontiguousarray(y), c, s, offset=0) if rot else y + y
         assert np.linalg.norm(got - want) <= 4e-3 * np.linalg.norm(want)
+
+
+def test_reversed_rows(gpu):
+    """A view with a negative row stride takes none of the kernels that form
+    unsigned offsets from the view's base."""
+    def flip(t):
+        return E.dispatchEager("reverse", [t], [("dimensions", "[0]")])[0]
+
+    r = np.random.default_rng(11)
+    for M, K, N in ((40, 256, 264), (2048, 64, 4096)):
+        x, w = _bf16(r, (M, K), 1.0), _bf16(r, (K, N), 0.05)
+        got = E.toHostF32(O.matmul(flip(_dev(x)), _dev(w)))
+        want = E.toHostF32(O.matmul(_dev(np.ascontiguousarray(x[::-1])), _dev(w)))
+        assert np.linalg.norm(got - want) <= 2e-3 * np.linalg.norm(want)
