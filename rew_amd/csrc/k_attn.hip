@@ -937,6 +937,287 @@ __global__ void __launch_bounds__(512, 1) flash_pp_kernel(FlashArgs a) {
 }
 
 
+// ---- few queries over many keys (a decode step) -----------------------------------
+//
+// A decode step has one query per head: the 128-query kernel runs it with
+// 127 empty columns, reads every K and V tile once per query head and gives
+// each (batch, head) to one workgroup however many keys there are.  Here the
+// Sq queries of all H / Hkv heads of one KV head (at most 32) are the 32
+// columns of one MFMA block, so K and V are read once, and the keys are
+// split over `splits` workgroups per KV head and the two waves of each.
+// What bounds it is the K / V stream: every wave owns its key tiles (64
+// keys, every second one) and two LDS stages for them, 32 KiB of K and V at
+// D = 128, one in flight by DMA while the other is used, so the waves need no
+// barriers and a CU keeps 64 KiB in flight.  Rows past Sk repeat the last
+// key (masked); past the last tile the DMA goes through a descriptor of
+// zero records and costs nothing.
+//
+// A wave's running max, sum and O (fp32) join the other wave's through LDS;
+// the workgroups' go to memory past the L2 (agent scope) and the last to
+// arrive merges them in split order, as in the strip GEMM.
+// 16 x 32 / 8 heads x 4000 keys x 128 (262 MB of K and V): 130 -> 57 us
+// (4.6 TB/s).
+namespace fa {
+constexpr int kDecCols = 32;
+constexpr int kDecMaxPairs = 4096;
+constexpr int64_t kDecWs = 4ll << 20;  // floats: partial O, then (max, sum) pairs
+constexpr int kAgent = 16;             // cache policy sc1: agent-scope access
+}  // namespace fa
+// (all launches of a device are ordered on its context's stream, and each
+// leaves the counts at zero)
+__device__ float g_dec_o[fa::kDecWs];
+__device__ float g_dec_ml[fa::kDecWs / 16];
+__device__ int g_dec_count[fa::kDecMaxPairs];
+
+template <int D, bool ROUND>
+__global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int splits, int per) {
+  using namespace fa;
+  constexpr int CPR = D / 8, NT = D / 16, DT = D / 32;
+  constexpr int TILE = BKV * D;
+  constexpr int RPD = 64 / CPR;     // key rows per 1 KiB DMA instruction
+  constexpr int NDMA = TILE / 512;  // instructions per K (or V) tile
+  __shared__ __attribute__((aligned(1024))) uint16_t S0[2 * 2 * TILE];
+  __shared__ __attribute__((aligned(1024))) uint16_t S1[2 * 2 * TILE];
+  typedef __attribute__((address_space(3))) uint16_t lds_u16;
+  typedef __attribute__((address_space(3))) float lds_f32;
+  typedef __attribute__((address_space(3))) bf16x8_t lds_bf16x8;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 31, g = lane >> 5;
+  const int pair = blockIdx.x / splits, split = blockIdx.x - pair * splits;
+  const int G = a.H / a.Hkv, rows = G * a.Sq;
+  const int b = pair / a.Hkv, hk = pair - b * a.Hkv;
+  const int cr = c < rows ? c : rows - 1;
+  const int h = hk * G + cr / a.Sq, qi = cr % a.Sq;
+  const int nkt = (a.Sk + BKV - 1) / BKV;
+  const int t0 = split * per + wave;                       // this wave's tiles: t0, t0 + 2, ..
+  const int n = max(0, (min(nkt, (split + 1) * per) - t0 + 1) / 2);
+
+  bf16x8_t qf[NT];
+  {
+    const uint16_t* qp = (const uint16_t*)a.q + b * a.q_sb + h * a.q_sh + (int64_t)qi * a.q_ss;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) qf[t] = *(const bf16x8_t*)(qp + t * 16 + g * 8);
+  }
+  const uint64_t K = (uint64_t)(uintptr_t)((const uint16_t*)a.k + b * a.k_sb + hk * a.k_sh);
+  const uint64_t V = (uint64_t)(uintptr_t)((const uint16_t*)a.v + b * a.v_sb + hk * a.v_sh);
+  auto rsrc = [](uint64_t p, uint32_t bytes) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)p);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)hi << 32) | lo),
+                                             (short)0, __builtin_amdgcn_readfirstlane((int)bytes),
+                                             0x00020000);
+  };
+  // the layouts of flash_fwd_kernel: chunk pc of key row r holds logical chunk
+  // pc ^ (r % CPR) of K and pc ^ (4 (r & 3)) of V
+  const int row_in = lane / CPR, pc = lane % CPR;
+  const uint32_t ks2 = (uint32_t)a.k_ss * 2, vs2 = (uint32_t)a.v_ss * 2;
+  auto dma_tile = [&](lds_u16* st, int i) {
+    const uint32_t bytes = i < n ? 0x7fffffffu : 0u;
+    const __amdgpu_buffer_rsrc_t rk = rsrc(K, bytes), rv = rsrc(V, bytes);
+    const int k0 = (t0 + 2 * i) * BKV;
+    lds_u16* sk = st + wave * 2 * TILE;
+#pragma unroll
+    for (int q = 0; q < NDMA; ++q) {
+      const int r = q * RPD + row_in;
+      const uint32_t key = (uint32_t)min(k0 + r, a.Sk - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void*)(sk + q * 512), 16,
+                                               key * ks2 + (uint32_t)((pc ^ (r % CPR)) * 16), 0, 0,
+                                               0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rv, (lds_void*)(sk + (TILE + q * 512)), 16,
+          key * vs2 + (uint32_t)((pc ^ ((4 * (r & 3)) % CPR)) * 16), 0, 0, 0);
+    }
+  };
+
+  int k_off[NT], v_off[DT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    k_off[t] = wave * 2 * TILE + c * D + (((2 * t + g) ^ (c % CPR)) * 8);
+    asm("" : "+v"(k_off[t]));
+  }
+  const int G16 = lane >> 4, s16 = lane & 15;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    const int r = 4 * (G16 >> 1) + (s16 >> 2);
+    const int col = dt * 32 + 16 * (G16 & 1) + 4 * (s16 & 3);
+    v_off[dt] = wave * 2 * TILE + TILE + r * D + (((col >> 3) ^ ((4 * (r & 3)) % CPR)) * 8) +
+                (col & 7);
+    asm("" : "+v"(v_off[dt]));
+  }
+
+  f32x16_t o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
+  float m_run = -INFINITY, l_run = 0.0f;
+  const float sl2 = a.scale * kLog2e;
+  const bool plain = !a.mask && a.scale > 0.0f;
+
+  auto compute = [&](lds_u16* st, int i) __attribute__((always_inline)) {
+    f32x16_t sacc[2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sacc[kb][e] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      sacc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(lds_bf16x8*)(st + k_off[t]), qf[t],
+                                                        sacc[0], 0, 0, 0);
+      sacc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(lds_bf16x8*)(st + (k_off[t] + 32 * D)),
+                                                        qf[t], sacc[1], 0, 0, 0);
+    }
+    uint32_t pk[2][8];
+    const float mr = fa_round_max<ROUND>(sacc);
+    const int k0 = (t0 + 2 * i) * BKV;
+    float alpha;
+    if (plain && k0 + BKV <= a.Sk)
+      fa_softmax_tile<DT, FA_PLAIN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    else
+      fa_softmax_tile<DT, FA_GENERAL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_rescale<DT>(o, alpha);
+    l_run = __fadd_rn(l_run, fa_row_sum(pk));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      union {
+        uint32_t w[4];
+        bf16x8_t v;
+      } pf;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) pf.w[x] = pk[u >> 1][(u & 1) * 4 + x];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        union {
+          v4s hh[2];
+          bf16x8_t v;
+        } vf;
+        vf.hh[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(st + (v_off[dt] + u * 16 * D)));
+        vf.hh[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_v4s*)(st + (v_off[dt] + (u * 16 + 8) * D)));
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf.v, o[dt], 0, 0, 0);
+      }
+    }
+  };
+  // tile i from stage st while tile i + 1 moves into the other one, whose
+  // reads are done
+  auto step = [&](lds_u16* st, lds_u16* next, int i) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    dma_tile(next, i + 1);
+    if constexpr (NDMA == 16) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
+    else if constexpr (NDMA == 8) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    compute(st, i);
+  };
+  dma_tile((lds_u16*)S0, 0);
+  int i = 0;
+  for (; i + 2 <= n; i += 2) {
+    step((lds_u16*)S0, (lds_u16*)S1, i);
+    step((lds_u16*)S1, (lds_u16*)S0, i + 1);
+  }
+  if (i < n) step((lds_u16*)S0, (lds_u16*)S1, i);
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __syncthreads();
+
+  // ---- join the two waves (through S0), then the splits ---------------------------
+  const auto lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run),
+                                                     false, false);
+  float l_tot = __uint_as_float(lsw[0]) + __uint_as_float(lsw[1]);
+  lds_f32* X = (lds_f32*)S0;
+  if (wave == 1) {
+    X[lane] = m_run;
+    X[64 + lane] = l_tot;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) X[128 + (dt * 16 + e) * 64 + lane] = o[dt][e];
+  }
+  __syncthreads();
+  lds_f32* F = X + 128 + DT * 16 * 64;  // the joined O, [32][D], then max and sum per column
+  if (wave == 0) {
+    const float m1 = X[lane];
+    const float m = fmaxf(m_run, m1);
+    const float mu = m == -INFINITY ? 0.0f : m;
+    const float w0 = fa_exp2(m_run - mu), w1 = fa_exp2(m1 - mu);
+    l_tot = l_tot * w0 + X[64 + lane] * w1;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        F[c * D + dt * 32 + (e >> 2) * 8 + g * 4 + (e & 3)] =
+            o[dt][e] * w0 + X[128 + (dt * 16 + e) * 64 + lane] * w1;
+    if (g == 0) {
+      F[32 * D + 2 * c] = m;
+      F[32 * D + 2 * c + 1] = l_tot;
+    }
+  }
+  __syncthreads();
+  auto store = [&](int r, int d, const float (&v)[4], float l) {
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    const int hh = hk * G + r / a.Sq, q = r % a.Sq;
+    uint16_t* O = (uint16_t*)a.o + b * a.o_sb + hh * a.o_sh + (int64_t)q * a.o_ss + d;
+    *(uint2*)O = make_uint2(cvt_bf16x2(v[0] * inv, v[1] * inv), cvt_bf16x2(v[2] * inv, v[3] * inv));
+  };
+  if (splits == 1) {
+    for (int x = tid * 4; x < rows * D; x += 512) {
+      const float v[4] = {F[x], F[x + 1], F[x + 2], F[x + 3]};
+      store(x / D, x % D, v, F[32 * D + 2 * (x / D) + 1]);
+    }
+    return;
+  }
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+  const __amdgpu_buffer_rsrc_t ro = rsrc((uint64_t)(uintptr_t)g_dec_o, (uint32_t)(kDecWs * 4));
+  const __amdgpu_buffer_rsrc_t rm = rsrc((uint64_t)(uintptr_t)g_dec_ml, (uint32_t)(kDecWs / 4));
+  const uint32_t first = (uint32_t)(pair * splits);
+  const uint32_t so = (uint32_t)(rows * D * 4), sm = (uint32_t)(rows * 8);  // bytes per split
+  for (int x = tid * 4; x < rows * D; x += 512) {
+    const u32x4_t v = {__float_as_uint(F[x]), __float_as_uint(F[x + 1]),
+                       __float_as_uint(F[x + 2]), __float_as_uint(F[x + 3])};
+    __builtin_amdgcn_raw_buffer_store_b128(v, ro, (uint32_t)x * 4, (first + split) * so, kAgent);
+  }
+  if (tid < rows) {
+    const u32x2_t v = {__float_as_uint(F[32 * D + 2 * tid]), __float_as_uint(F[32 * D + 2 * tid + 1])};
+    __builtin_amdgcn_raw_buffer_store_b64(v, rm, (uint32_t)tid * 8, (first + split) * sm, kAgent);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  __attribute__((address_space(3))) int* last = (__attribute__((address_space(3))) int*)S1;
+  if (tid == 0) {
+    const int k = __hip_atomic_fetch_add(&g_dec_count[pair], 1, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+    *last = k == splits - 1;
+    if (k == splits - 1)
+      __hip_atomic_store(&g_dec_count[pair], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!*last) return;
+  for (int x = tid * 4; x < rows * D; x += 512) {
+    const int r = x / D;
+    float m = -INFINITY;
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s)
+      m = fmaxf(m, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                       rm, (uint32_t)r * 8, (first + s) * sm, kAgent)));
+    const float mu = m == -INFINITY ? 0.0f : m;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, l = 0.0f;
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s) {
+      const u32x2_t ml =
+          __builtin_amdgcn_raw_buffer_load_b64(rm, (uint32_t)r * 8, (first + s) * sm, kAgent);
+      const u32x4_t v =
+          __builtin_amdgcn_raw_buffer_load_b128(ro, (uint32_t)x * 4, (first + s) * so, kAgent);
+      const float w = fa_exp2(__uint_as_float(ml[0]) - mu);
+      l += __uint_as_float(ml[1]) * w;
+#pragma unroll
+      for (int y = 0; y < 4; ++y) acc[y] += __uint_as_float(v[y]) * w;
+    }
+    store(r, x % D, acc, l);
+  }
+}
+
 bool flash_supported(const FlashArgs& a) {
   if (a.D != 32 && a.D != 64 && a.D != 128) return false;
   if (a.B <= 0 || a.H <= 0 || a.Hkv <= 0 || a.H % a.Hkv) return false;
@@ -967,7 +1248,7 @@ static void launch_flash_d(const FlashArgs& a, bool buf, unsigned grid, hipStrea
 // every K / V byte offset fits the buffer descriptors' 31 bits; other
 // shapes run the single-group kernel.  REW_MI355X_FLASH = single or pp
 // forces one (tests compare them).
-enum { FA_K_SINGLE = 0, FA_K_PP = 1 };
+enum { FA_K_SINGLE = 0, FA_K_PP = 1, FA_K_DEC = 2 };
 static int flash_forced() {
   static const int v = [] {
     const char* s = std::getenv("REW_MI355X_FLASH");
@@ -983,7 +1264,46 @@ static bool flash_buf_ok(const FlashArgs& a) {
          ((int64_t)a.Sk * a.v_ss + a.D) * 2 < (1ll << 31);
 }
 
+// Few queries per KV head (at most the 32 columns of a block) and keys enough
+// for a tile per wave.  With one query head per KV head there is nothing to
+// share, and the 128-query kernel, four waves on each tile, streams as fast
+// once its workgroups fill half of the CUs (32 x 32 / 32 heads x 1000 keys:
+// 103 us against 108); with two or more this one was ahead at every size
+// measured (64 x 32 / 8 heads x 300 keys 53 -> 28 us, 16 x 32 / 8 heads x 128
+// keys 10.9 -> 9.1).
+static bool flash_dec_ok(const FlashArgs& a) {
+  const int64_t pairs = (int64_t)a.B * a.Hkv;
+  const bool fill = a.H > a.Hkv || (pairs <= 128 && a.Sk >= 8 * fa::BKV);
+  return fill && (int64_t)(a.H / a.Hkv) * a.Sq <= fa::kDecCols && a.Sk >= 2 * fa::BKV &&
+         pairs < (1 << 20) && a.k_ss >= 0 && a.v_ss >= 0 &&
+         ((int64_t)a.Sk * a.k_ss + a.D) * 2 < (1ll << 31) &&
+         ((int64_t)a.Sk * a.v_ss + a.D) * 2 < (1ll << 31);
+}
+
+// Key tiles per split: the fewest rounds of tiles over the CUs (two waves a
+// workgroup; at D = 128 one workgroup a CU, else two), a merge counted as one
+// more and another for each eight columns it reads.
+static void flash_dec_plan(const FlashArgs& a, int* splits, int* per) {
+  const int64_t pairs = (int64_t)a.B * a.Hkv, rows = (int64_t)(a.H / a.Hkv) * a.Sq;
+  const int64_t nkt = (a.Sk + fa::BKV - 1) / fa::BKV, slots = a.D == 128 ? 256 : 512;
+  int64_t best = 1ll << 60;
+  for (int64_t s = 1; s <= 64 && s <= nkt; ++s) {
+    if (s > 1 && (pairs > fa::kDecMaxPairs || pairs * s * rows * a.D > fa::kDecWs ||
+                  pairs * s * rows * 2 > fa::kDecWs / 16))
+      break;
+    const int64_t p = (nkt + s - 1) / s, n = (nkt + p - 1) / p;
+    const int64_t cost = ((pairs * n + slots - 1) / slots) * ((p + 1) / 2) +
+                         (n > 1 ? 1 + rows / 8 : 0);
+    if (cost < best) {
+      best = cost;
+      *splits = (int)n;
+      *per = (int)p;
+    }
+  }
+}
+
 static int flash_kernel_kind(const FlashArgs& a) {
+  if (flash_forced() < 0 && flash_dec_ok(a)) return FA_K_DEC;
   if (!((a.D == 64 || a.D == 128) && flash_buf_ok(a))) return FA_K_SINGLE;
   const int f = flash_forced();
   return f >= 0 ? f : FA_K_PP;
@@ -992,6 +1312,7 @@ static int flash_kernel_kind(const FlashArgs& a) {
 const char* flash_variant(const FlashArgs& a) {
   switch (flash_kernel_kind(a)) {
     case FA_K_PP: return "flash_attn_pp";
+    case FA_K_DEC: return "flash_attn_dec";
     default: return "flash_attn";
   }
 }
@@ -999,6 +1320,26 @@ const char* flash_variant(const FlashArgs& a) {
 void launch_flash(const FlashArgs& a, hipStream_t stream) {
   const int nqt = (a.Sq + fa::BQ - 1) / fa::BQ;
   const int kind = flash_kernel_kind(a);
+  if (kind == FA_K_DEC) {
+    int splits = 1, per = 1;
+    flash_dec_plan(a, &splits, &per);
+    const unsigned grid = (unsigned)(a.B * a.Hkv * splits);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(128), 0, stream, a, splits, per);
+    };
+    if (a.D == 32) {
+      if (a.round_scores) go(flash_dec_kernel<32, true>);
+      else go(flash_dec_kernel<32, false>);
+    } else if (a.D == 64) {
+      if (a.round_scores) go(flash_dec_kernel<64, true>);
+      else go(flash_dec_kernel<64, false>);
+    } else {
+      if (a.round_scores) go(flash_dec_kernel<128, true>);
+      else go(flash_dec_kernel<128, false>);
+    }
+    REW_HIP(hipGetLastError());
+    return;
+  }
   if (kind == FA_K_PP) {
     const bool pair = ((a.H / a.Hkv) & 1) == 0;
     const unsigned grid =
