@@ -133,6 +133,11 @@ __device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t r, uint32_t vof
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voff, soff, 0, 0);
 }
 
+__device__ __forceinline__ void dma16_lds(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
+                                          lds_void* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds, 16, voff, soff, 0, 0);
+}
+
 // Tile kinds of the softmax step, each straight-line code:
 //   0 plain     every key in range and visible, scale > 0: t is formed
 //               inside the exp's FMA and the max comes from the raw
@@ -140,7 +145,10 @@ __device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t r, uint32_t vof
 //   1 diagonal  a whole tile under an ordered mask that adds 0 where
 //               visible, scale > 0: t = fma(x, scale log2 e, visible ? 0 :
 //               mask_false log2 e), visibility from one per-lane threshold;
-//   2 general   anything else: t = (x * scale + mask) log2 e, -inf past Sk.
+//   2 general   anything else: t = (x * scale + mask) log2 e, -inf past Sk
+//               and below jlo, from which a ragged last tile that was moved
+//               back to end at Sk counts its keys;
+//   4 tail      such a tile without a mask, scale > 0: -inf below jlo.
 // The plain tiles of queries [q0, q_last] form one range of key tiles
 // [lo, hi), found once per wave group instead of per tile.
 struct FaKinds {
@@ -208,9 +216,9 @@ __device__ __forceinline__ float fa_round_max(f32x16_t (&sacc)[2]) {
 // PV product (the running sum is left to fa_row_sum).  One straight-line body per tile
 // kind (FA_PLAIN, FA_DIAG_UP / FA_DIAG_DOWN for masks that keep keys above /
 // below the diagonal, FA_GENERAL).
-enum { FA_PLAIN = 0, FA_DIAG_UP = 1, FA_GENERAL = 2, FA_DIAG_DOWN = 3 };
+enum { FA_PLAIN = 0, FA_DIAG_UP = 1, FA_GENERAL = 2, FA_DIAG_DOWN = 3, FA_TAIL = 4 };
 template <int DT, int KIND>
-__device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int qi, int g,
+__device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int jlo, int qi, int g,
                                                 float sl2, f32x16_t (&sacc_in)[2],
                                                 float mr, uint32_t (&pk)[2][8], float& m_run,
                                                 float& l_run, float& alpha_out) {
@@ -219,14 +227,15 @@ __device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int 
   float mt;
   if constexpr (KIND == FA_PLAIN) {
     mt = mr * sl2;
-  } else if constexpr (KIND == FA_DIAG_UP || KIND == FA_DIAG_DOWN) {
+  } else if constexpr (KIND == FA_DIAG_UP || KIND == FA_DIAG_DOWN || KIND == FA_TAIL) {
     // key j = k0 + off (off = kb 32 + (e / 4) 8 + g 4 + e % 4) is visible
     // iff j - qi >= lo (LE, LT) or j - qi <= -lo (GE, GT)
-    constexpr bool kUp = KIND == FA_DIAG_UP;
-    const float mf2 = a.mask_false * kLog2e;
+    // (tail: j >= jlo, and -inf below)
+    constexpr bool kUp = KIND != FA_DIAG_DOWN;
+    const float mf2 = KIND == FA_TAIL ? -INFINITY : a.mask_false * kLog2e;
     const int lo = (a.cmp == vm::CMP_LT || a.cmp == vm::CMP_GT) ? 1 : 0;
     const int base = k0 - qi + g * 4;
-    const int thr = kUp ? lo - base : -lo - base;
+    const int thr = KIND == FA_TAIL ? jlo - k0 - g * 4 : kUp ? lo - base : -lo - base;
     float m0 = -INFINITY, m1 = -INFINITY;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -255,8 +264,8 @@ __device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int 
           x0 += fa_visible(a.cmp, qi, j0) ? a.mask_true : a.mask_false;
           x1 += fa_visible(a.cmp, qi, j0 + 1) ? a.mask_true : a.mask_false;
         }
-        x0 = j0 < a.Sk ? x0 * kLog2e : -INFINITY;
-        x1 = j0 + 1 < a.Sk ? x1 * kLog2e : -INFINITY;
+        x0 = j0 >= jlo && j0 < a.Sk ? x0 * kLog2e : -INFINITY;
+        x1 = j0 + 1 >= jlo && j0 + 1 < a.Sk ? x1 * kLog2e : -INFINITY;
         t[kb][e] = x0;
         t[kb][e + 1] = x1;
         m0 = fmaxf(m0, fmaxf(x0, x1));
@@ -326,19 +335,19 @@ __device__ __forceinline__ float fa_row_sum(const uint32_t (&pk)[2][8]) {
 
 // The softmax step of the tile's kind (fa_kind), then the rescale of O.
 template <int DT>
-__device__ __forceinline__ void fa_softmax_any(int kind, const FlashArgs& a, int k0, int qi,
-                                               int g, float sl2, f32x16_t (&sacc)[2],
+__device__ __forceinline__ void fa_softmax_any(int kind, const FlashArgs& a, int k0, int jlo,
+                                               int qi, int g, float sl2, f32x16_t (&sacc)[2],
                                                float mr, uint32_t (&pk)[2][8], f32x16_t (&o)[DT],
                                                float& m_run, float& l_run) {
   float alpha;
   if (kind == FA_PLAIN)
-    fa_softmax_tile<DT, FA_PLAIN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_PLAIN>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   else if (kind == FA_DIAG_UP)
-    fa_softmax_tile<DT, FA_DIAG_UP>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_DIAG_UP>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   else if (kind == FA_DIAG_DOWN)
-    fa_softmax_tile<DT, FA_DIAG_DOWN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_DIAG_DOWN>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   else
-    fa_softmax_tile<DT, FA_GENERAL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_GENERAL>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   fa_rescale<DT>(o, alpha);
 }
 
@@ -354,8 +363,9 @@ __device__ __forceinline__ void block_barrier_fa() {
   asm volatile("" ::: "memory");
 }
 
-// BUF: every key tile is whole (Sk % 64 == 0) and every byte offset into K
-// and V is below 2^31, so the tiles move by buffer loads with a scalar tile
+// BUF: at least one whole key tile (a ragged last one is moved back to end at
+// Sk and drops the keys it repeats) and every byte offset into K and V below
+// 2^31, so the tiles move by buffer loads with a scalar tile
 // offset (no per-tile address arithmetic on the vector ALU).
 // ROUND: scores are rounded to bf16 before the scale (a.round_scores).
 template <int D, bool BUF, bool ROUND>
@@ -443,7 +453,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
     }
   }
   auto dma_tile = [&](uint16_t* ks, uint16_t* vs, int kt) {
-    const int k0 = kt * BKV;
+    const int k0 = BUF ? min(kt * BKV, a.Sk - BKV) : kt * BKV;
     if constexpr (BUF) {
       const uint32_t sk = (uint32_t)(k0 * a.k_ss * 2), sv = (uint32_t)(k0 * a.v_ss * 2);
 #pragma unroll
@@ -548,7 +558,8 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
     const int k0 = kt * BKV;
     uint32_t pk[2][8];  // bf16 probability pairs: [kb][e/2]
     const float mr = fa_round_max<ROUND>(sacc);
-    fa_softmax_any<DT>(fa_kind(kinds, kt), a, k0, qi, g, sl2, sacc, mr, pk, o, m_run, l_run);
+    fa_softmax_any<DT>(fa_kind(kinds, kt), a, BUF ? min(k0, a.Sk - BKV) : k0, k0, qi, g, sl2, sacc,
+                       mr, pk, o, m_run, l_run);
     l_run = __fadd_rn(l_run, fa_row_sum(pk));
 
     // O^T += V^T P^T over 4 k-steps of 16 keys
@@ -834,7 +845,8 @@ __global__ void __launch_bounds__(512, 1) flash_pp_kernel(FlashArgs a) {
   float mr = -INFINITY;  // max of the rounded scores of the last S tile
   auto soft_phase = [&](int m) {
     const int k0 = (kt0 + m) * BKV;
-    fa_softmax_any<DT>(fa_kind(kinds, kt0 + m), a, k0, qi, g, sl2, sacc, mr, pk, o, m_run, l_run);
+    fa_softmax_any<DT>(fa_kind(kinds, kt0 + m), a, k0, k0, qi, g, sl2, sacc, mr, pk, o, m_run,
+                       l_run);
   };
   // the MFMA phase's share of the softmax: the scores' rounding and max,
   // and the row sum of the last probabilities (in the softmax phase instead
@@ -948,15 +960,15 @@ __global__ void __launch_bounds__(512, 1) flash_pp_kernel(FlashArgs a) {
 // What bounds it is the K / V stream: every wave owns its key tiles (64
 // keys, every second one) and two LDS stages for them, 32 KiB of K and V at
 // D = 128, one in flight by DMA while the other is used, so the waves need no
-// barriers and a CU keeps 64 KiB in flight.  Rows past Sk repeat the last
-// key (masked); past the last tile the DMA goes through a descriptor of
+// barriers and a CU keeps 64 KiB in flight.  A ragged last tile is moved back
+// to end at Sk; past the last tile the DMA goes through a descriptor of
 // zero records and costs nothing.
 //
 // A wave's running max, sum and O (fp32) join the other wave's through LDS;
 // the workgroups' go to memory past the L2 (agent scope) and the last to
 // arrive merges them in split order, as in the strip GEMM.
-// 16 x 32 / 8 heads x 4000 keys x 128 (262 MB of K and V): 130 -> 57 us
-// (4.6 TB/s).
+// 16 x 32 / 8 heads x 4000 keys x 128 (262 MB of K and V): 130 -> 54 us
+// (4.9 TB/s).
 namespace fa {
 constexpr int kDecCols = 32;
 constexpr int kDecMaxPairs = 4096;
@@ -1011,22 +1023,23 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
   // the layouts of flash_fwd_kernel: chunk pc of key row r holds logical chunk
   // pc ^ (r % CPR) of K and pc ^ (4 (r & 3)) of V
   const int row_in = lane / CPR, pc = lane % CPR;
-  const uint32_t ks2 = (uint32_t)a.k_ss * 2, vs2 = (uint32_t)a.v_ss * 2;
+  uint32_t kv_off[NDMA], vv_off[NDMA];
+#pragma unroll
+  for (int q = 0; q < NDMA; ++q) {
+    const int r = q * RPD + row_in;
+    kv_off[q] = (uint32_t)((r * a.k_ss + (pc ^ (r % CPR)) * 8) * 2);
+    vv_off[q] = (uint32_t)((r * a.v_ss + (pc ^ ((4 * (r & 3)) % CPR)) * 8) * 2);
+  }
   auto dma_tile = [&](lds_u16* st, int i) {
     const uint32_t bytes = i < n ? 0x7fffffffu : 0u;
     const __amdgpu_buffer_rsrc_t rk = rsrc(K, bytes), rv = rsrc(V, bytes);
-    const int k0 = (t0 + 2 * i) * BKV;
-    lds_u16* sk = st + wave * 2 * TILE;
+    const int k0 = i < n ? min((t0 + 2 * i) * BKV, a.Sk - BKV) : 0;
+    const uint32_t sk = (uint32_t)(k0 * a.k_ss * 2), sv = (uint32_t)(k0 * a.v_ss * 2);
+    lds_u16* sd = st + wave * 2 * TILE;
 #pragma unroll
     for (int q = 0; q < NDMA; ++q) {
-      const int r = q * RPD + row_in;
-      const uint32_t key = (uint32_t)min(k0 + r, a.Sk - 1);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void*)(sk + q * 512), 16,
-                                               key * ks2 + (uint32_t)((pc ^ (r % CPR)) * 16), 0, 0,
-                                               0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rv, (lds_void*)(sk + (TILE + q * 512)), 16,
-          key * vs2 + (uint32_t)((pc ^ ((4 * (r & 3)) % CPR)) * 16), 0, 0, 0);
+      dma16_lds(rk, kv_off[q], sk, (lds_void*)(sd + q * 512));
+      dma16_lds(rv, vv_off[q], sv, (lds_void*)(sd + (TILE + q * 512)));
     }
   };
 
@@ -1072,10 +1085,13 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
     const float mr = fa_round_max<ROUND>(sacc);
     const int k0 = (t0 + 2 * i) * BKV;
     float alpha;
-    if (plain && k0 + BKV <= a.Sk)
-      fa_softmax_tile<DT, FA_PLAIN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    const int kb0 = min(k0, a.Sk - BKV);
+    if (plain && k0 == kb0)
+      fa_softmax_tile<DT, FA_PLAIN>(a, kb0, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    else if (plain)
+      fa_softmax_tile<DT, FA_TAIL>(a, kb0, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     else
-      fa_softmax_tile<DT, FA_GENERAL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+      fa_softmax_tile<DT, FA_GENERAL>(a, kb0, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     fa_rescale<DT>(o, alpha);
     l_run = __fadd_rn(l_run, fa_row_sum(pk));
 #pragma unroll
@@ -1246,7 +1262,9 @@ static void launch_flash_d(const FlashArgs& a, bool buf, unsigned grid, hipStrea
 
 // Kernel choice for head dims 64 and 128 when every key tile is whole and
 // every K / V byte offset fits the buffer descriptors' 31 bits; other
-// shapes run the single-group kernel.  REW_MI355X_FLASH = single or pp
+// shapes run the single-group kernel (ragged key counts through ping-pong,
+// the last tile moved back, measured 5 to 50 % slower below 1500 keys: half
+// the workgroups, and the mask's tile in the longer general form).  REW_MI355X_FLASH = single or pp
 // forces one (tests compare them).
 enum { FA_K_SINGLE = 0, FA_K_PP = 1, FA_K_DEC = 2 };
 static int flash_forced() {
@@ -1260,7 +1278,7 @@ static int flash_forced() {
 }
 
 static bool flash_buf_ok(const FlashArgs& a) {
-  return a.Sk % fa::BKV == 0 && ((int64_t)a.Sk * a.k_ss + a.D) * 2 < (1ll << 31) &&
+  return a.k_ss >= 0 && a.v_ss >= 0 && ((int64_t)a.Sk * a.k_ss + a.D) * 2 < (1ll << 31) &&
          ((int64_t)a.Sk * a.v_ss + a.D) * 2 < (1ll << 31);
 }
 
@@ -1304,7 +1322,7 @@ static void flash_dec_plan(const FlashArgs& a, int* splits, int* per) {
 
 static int flash_kernel_kind(const FlashArgs& a) {
   if (flash_forced() < 0 && flash_dec_ok(a)) return FA_K_DEC;
-  if (!((a.D == 64 || a.D == 128) && flash_buf_ok(a))) return FA_K_SINGLE;
+  if (!((a.D == 64 || a.D == 128) && a.Sk % fa::BKV == 0 && flash_buf_ok(a))) return FA_K_SINGLE;
   const int f = flash_forced();
   return f >= 0 ? f : FA_K_PP;
 }
@@ -1358,7 +1376,7 @@ void launch_flash(const FlashArgs& a, hipStream_t stream) {
     return;
   }
   const unsigned grid = (unsigned)(nqt * a.B * a.H);
-  const bool buf = flash_buf_ok(a);
+  const bool buf = a.Sk >= fa::BKV && flash_buf_ok(a);
   switch (a.D) {
     case 32: launch_flash_d<32>(a, buf, grid, stream); break;
     case 64: launch_flash_d<64>(a, buf, grid, stream); break;
