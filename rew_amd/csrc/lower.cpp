@@ -325,6 +325,7 @@ struct Lower {
   std::unordered_map<Tensor*, MoePlan> moe_out;
   std::unordered_map<Tensor*, Node*> flash_out;  // transposed flash output -> PV node
   std::unordered_map<Tensor*, HeadPlan> head_out;  // argmax output -> fused head
+  std::unordered_map<Tensor*, HeadPlan> head_probs;  // softmax output -> fused Linear + softmax
   std::unordered_map<Tensor*, RouterPlan> router_out;  // its ids / weights / values -> router
   std::vector<std::vector<Tensor*>> gemm_groups;  // outputs of sibling projections
   // reductions emitted in this flush, by (input, op, dims, dtype): a repeat
@@ -352,7 +353,7 @@ struct Lower {
   bool plan_norm(NormPlan np, Tensor* x, int x_uses, Tensor* o, std::vector<Tensor*>& inner);
   bool match_layernorm(Node* ao);
   void match_class_head();
-  bool emit_class_head(Node* n, const HeadPlan& p);
+  bool emit_class_head(Tensor* probs, Tensor* ids, const HeadPlan& p);
   void match_router();
   bool emit_router(const RouterPlan& p);
   bool emit_norm(Tensor* t, const NormPlan& p);
@@ -962,6 +963,12 @@ void Lower::ensure_mat(Tensor* t) {
   if (sit != softmax_out.end()) {
     SoftmaxPlan sp = sit->second;
     softmax_out.erase(sit);
+    auto hit = head_probs.find(t);
+    if (hit != head_probs.end()) {
+      const HeadPlan hp = hit->second;
+      head_probs.erase(hit);
+      if (emit_class_head(t, nullptr, hp)) return;
+    }
     if (emit_softmax(t, sp)) return;
   }
   auto fit = flash_out.find(t);
@@ -3073,7 +3080,7 @@ void Lower::emit_argmax(Node* n) {
   if (hit != head_out.end()) {
     const HeadPlan hp = hit->second;
     head_out.erase(hit);
-    if (emit_class_head(n, hp)) return;
+    if (emit_class_head(nullptr, out, hp)) return;
     // outside the fused kernel's limits: the head runs as its own kernels
   }
   ensure_mat(x);
@@ -3095,38 +3102,65 @@ void Lower::emit_argmax(Node* n) {
   run_launch(c, std::move(L));
 }
 
-// The classifier head: an argmax over dim 1 of a planned softmax of a
-// planned Linear (bias epilogue) whose logits and probabilities have no
-// other reader.  The plans stay registered, so a head the fused kernel
-// cannot take is emitted by them instead.
+// The classifier head: a planned softmax over dim 1 of a planned Linear (bias
+// epilogue) whose logits have no other reader, and an argmax of the
+// probabilities where nothing else reads those.  The plans stay registered,
+// so a head the fused kernel cannot take is emitted by them instead.
 void Lower::match_class_head() {
+  auto head = [&](Tensor* p, HeadPlan* hp) {
+    if (p->dt != kF32 || p->shape.rank != 2 || p->st) return false;
+    auto sit = softmax_out.find(p);
+    if (sit == softmax_out.end()) return false;
+    Tensor* lg = sit->second.x;
+    auto lit = gemm_out.find(lg);
+    if (lit == gemm_out.end() || lg->st || lg->ext != 0 || lg->uses != 2) return false;
+    const GemmPlan& lp = lit->second;
+    if (lp.epi != EPI_BIAS || lp.dot2 || lp.group >= 0 || lg->shape != p->shape) return false;
+    Tensor *x = lp.dot->in[0], *w = lp.dot->in[1];
+    if (x->dt != kF32 || w->dt != kF32 || lg->dt != kF32 || lp.bias->dt != kF32) return false;
+    hp->x = x;
+    hp->w = w;
+    hp->b = lp.bias;
+    return true;
+  };
   for (Node* n : nodes) {
     if (n->kind != K_ARGMAX || n->i0 != 1) continue;
     Tensor* p = n->in[0];
-    if (p->dt != kF32 || p->shape.rank != 2 || p->st || p->ext != 0 || p->uses != 1) continue;
-    auto sit = softmax_out.find(p);
-    if (sit == softmax_out.end()) continue;
-    Tensor* lg = sit->second.x;
-    auto lit = gemm_out.find(lg);
-    if (lit == gemm_out.end() || lg->st || lg->ext != 0 || lg->uses != 2) continue;
-    const GemmPlan& lp = lit->second;
-    if (lp.epi != EPI_BIAS || lp.dot2 || lp.group >= 0 || lg->shape != p->shape) continue;
-    Tensor *x = lp.dot->in[0], *w = lp.dot->in[1];
-    if (x->dt != kF32 || w->dt != kF32 || lg->dt != kF32 || lp.bias->dt != kF32) continue;
     HeadPlan hp;
-    hp.x = x;
-    hp.w = w;
-    hp.b = lp.bias;
+    if (p->ext != 0 || p->uses != 1 || !head(p, &hp)) continue;
     head_out[n->out[0]] = hp;
-    lg->plan_mat = false;
+    softmax_out[p].x->plan_mat = false;
     p->plan_mat = false;
+  }
+  for (auto& so : softmax_out) {
+    Tensor* p = so.first;
+    HeadPlan hp;
+    if (!p->plan_mat || !so.second.x->plan_mat) continue;
+    // Where the probabilities are stored the fused kernel replaces a product
+    // and a softmax of two launches.  Every workgroup (4 rows) stages the
+    // whole weight again, so it wins while the chip holds the workgroups at
+    // once and falls behind after that: [rows, inputs, classes] fused against
+    // the two kernels 128x128x10 7.5 us / 15.1, 512x512x10 9.6 / 23.5,
+    // 2048x128x60 11.4 / 22.8, but 2048x1000x8 18.0 / 17.6, 8192x128x10
+    // 15.3 / 17.2, 8192x128x60 26.4 / 25.5, 32768x128x10 43 / 22.
+    const int64_t M = p->shape.d[0];
+    if (M > 2048 || !head(p, &hp)) continue;
+    HeadArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.x = reinterpret_cast<const float*>(uintptr_t(256));
+    a.M = M;
+    a.K = hp.x->shape.d[1];
+    a.N = p->shape.d[1];
+    if (!class_head_ok(a) || (M > 1024 && a.K > 256)) continue;
+    so.second.x->plan_mat = false;
+    head_probs[p] = hp;
   }
 }
 
-bool Lower::emit_class_head(Node* n, const HeadPlan& p) {
-  Tensor* out = n->out[0];
+bool Lower::emit_class_head(Tensor* probs, Tensor* ids, const HeadPlan& p) {
   const int64_t M = p.x->shape.d[0], K = p.x->shape.d[1], N = p.w->shape.d[1];
-  if (p.w->shape.d[0] != K || out->numel() != M) return false;
+  if (p.w->shape.d[0] != K || (ids && ids->numel() != M) || (probs && probs->numel() != M * N))
+    return false;
   // a dense [rows, cols] (or [cols]) f32 operand's address, or null
   auto dense = [&](Tensor* t, int64_t cols) -> const float* {
     Tensor* base;
@@ -3149,8 +3183,15 @@ bool Lower::emit_class_head(Node* n, const HeadPlan& p) {
   a.w = dense(p.w, N);
   a.b = dense(p.b, N);
   if (!a.w || !a.b || !class_head_ok(a)) return false;
-  tensor_alloc(out);
-  a.ids = (int32_t*)out->data();
+  if (probs && ((uintptr_t)a.w & 15)) return false;  // (its weight is read in 16-byte loads)
+  if (ids) {
+    tensor_alloc(ids);
+    a.ids = (int32_t*)ids->data();
+  }
+  if (probs) {
+    tensor_alloc(probs);
+    a.probs = (float*)probs->data();
+  }
   Launch L{a};
   if (c->profiling)
     L.name = "class_head{" + std::to_string(M) + "x" + std::to_string(K) + "x" +

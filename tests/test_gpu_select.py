@@ -127,6 +127,41 @@ def test_mlp_forward_two_launches(gpu, oracle, M, K, N1, N2, fused):
     np.testing.assert_array_equal(ids, want)
 
 
+@pytest.mark.parametrize("M,K,N,fused", [(1, 4, 1, True), (5, 128, 64, True), (1024, 260, 10, True),
+                                         (1025, 260, 10, False), (2047, 256, 31, True),
+                                         (2049, 64, 3, False), (9, 1024, 8, True),
+                                         (9, 1024, 9, False), (9, 30, 4, False)])
+def test_softmax_of_linear_one_launch(gpu, oracle, M, K, N, fused):
+    """softmax(Linear(x)) read without an argmax runs in one launch within
+    the head kernel's limits and the two kernels past them; the probabilities
+    equal those of the two kernels bit for bit, from whole rows and from
+    every second one."""
+    rs = np.random.default_rng(M + K + N)
+    x = rs.standard_normal((2 * M, K)).astype(np.float32)
+    if M > 4:
+        x[4, 1] = np.nan
+    xt, lin = dev(x), nn.Linear(dev(rs.standard_normal((K, N)).astype(np.float32)),
+                                dev(rs.standard_normal(N).astype(np.float32)))
+    for xs, xh in ((O.slice_(xt, [0, 0], [M, K], [1, 1]), x[:M]),
+                   (O.slice_(xt, [0, 0], [2 * M, K], [2, 1]), x[::2])):
+        E.profileBegin()
+        got = E.toHost(nn.softmax(lin.forward(xs), 1))
+        names = [n for n, _, _ in E.profileEnd()]
+        assert (names == [f"class_head{{{M}x{K}x{N}}}"]) == fused, names
+        z = lin.forward(xs)
+        E.toHost(z)
+        np.testing.assert_array_equal(got, E.toHost(nn.softmax(z, 1)))
+        # (a chain of K fmas and the bias in f32: each logit within (K + 1)
+        # half-ulps of the terms' magnitudes)
+        w64, b64 = E.toHost(lin.weight).astype(np.float64), E.toHost(lin.bias)
+        ok = ~np.isnan(xh).any(1)
+        z64 = xh[ok].astype(np.float64) @ w64 + b64
+        tol = 2.0**-23 * (K + 1) * (np.abs(xh[ok]) @ np.abs(w64) + np.abs(b64)).max() + 1e-6
+        p64 = np.exp(z64 - z64.max(1, keepdims=True))
+        np.testing.assert_allclose(got[ok], p64 / p64.sum(1, keepdims=True), rtol=2 * tol, atol=1e-30)
+        assert np.isnan(got[~ok]).all()
+
+
 def test_mnist_mlp_inference(gpu, oracle):
     """Config C1: x [128,784] ~ U[0,1); Linear 784->128 + relu, Linear 128->10,
     softmax, argmax; Glorot-uniform weights (nn/init.nim:93-97), zero biases."""
