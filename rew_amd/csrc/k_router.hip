@@ -6,11 +6,14 @@
 //   topWeights = topW / reduceSum(topW, [1])
 // The logits, probabilities and unnormalised values never reach memory.
 //
-// The product is gemm_f32_narrow_kernel's (16 rows per workgroup, thread t
-// owns row t / 16 and columns 4 (t % 16) .. + 3, 32-deep k-steps in two
-// register sets): every logit is the same sequential fmaf chain over k from
-// 0, then the bias add.  For H % 128 == 0 the matrix-core form below runs
-// the same chains on f32 MFMAs, which round each step as fmaf does.  x may
+// Every logit is the same sequential fmaf chain over k from 0, then the bias
+// add, in one of three forms.  Up to 2048 tokens one or two rows take a wave
+// (the row form: a chain's latency is all there is, and the chip has a SIMD
+// for each).  Past that the matrix-core form, for H % 128 == 0, runs the
+// chains on f32 MFMAs, which round each step as fmaf does, and other H take
+// gemm_f32_narrow_kernel's product (16 rows per workgroup, thread t owns row
+// t / 16 and columns 4 (t % 16) .. + 3, 32-deep k-steps in two register
+// sets).  x may
 // be bf16: its conversion to f32 is exact and happens on the load.  Then
 // the 16 lanes of each row take
 // softmax_tile_kernel's steps (the max, expf, the running sum in column
@@ -120,6 +123,193 @@ __device__ __forceinline__ void router_tail(const RouterArgs& a, float (&y)[COLS
   }
   if (l == 0 && row_ok && a.weights)
     for (int s = 0; s < a.k; ++s) a.weights[t * a.k + s] = lg[s] / denom;
+}
+
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+typedef __attribute__((address_space(3))) float lds_f32;
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) u32x4_t lds_u32x4;
+
+// (buffer loads: with global ones the compiler waits for every LDS read at
+// the first use of any)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t router_rsrc(const void* base, uint32_t bytes) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  void* p = (void*)(uintptr_t)(((uint64_t)hi << 32) | lo);
+  return __builtin_amdgcn_make_buffer_rsrc(p, (short)0,
+                                           (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+__device__ __forceinline__ void router_dma(__amdgpu_buffer_rsrc_t r, uint32_t voff, lds_u8* lds) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voff, 0, 0, 0);
+}
+
+// s_waitcnt's field for `vm` vector-memory operations left in flight, every
+// LDS operation done
+constexpr int router_wait(int vm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4); }
+
+// The row form.  Wave w of W owns rows R w .. R w + R - 1 of the workgroup's
+// W R, lane l column l.  A logit is H dependent multiply-adds whatever the
+// form: here a step takes about 7 ns (in the matrix-core form, where a wave
+// alternates between two chains of dependent MFMAs, about 19).  W comes
+// through LDS, read by every wave for itself, so with four waves per CU the
+// LDS reads weigh as much as the chain; up to 512 tokens each row has a
+// workgroup of its own instead.  x is read as an LDS broadcast; as a DPP
+// operand of the multiply-add it was slower from four rows per wave on (8192
+// tokens 72 us against the matrix-core form's 50), DPP running at half rate.  A chunk of 64 k (W's rows padded to 64 columns, and each wave's
+// rows of x) is a stage of a four-deep LDS ring filled by DMA; a stage is ND
+// DMA instructions per wave.
+template <bool XBF16, int R, int W>
+__global__ void __launch_bounds__(64 * W, 1) moe_router_row_kernel(RouterArgs a) {
+  constexpr int NS = 4;
+  constexpr int XE = XBF16 ? 2 : 4;
+  constexpr int RPI = 16 / XE;  // rows of x in one DMA instruction
+  constexpr int NW = 16 / W;    // DMA instructions of W per wave
+  constexpr int STAGE = 16384 + W * 1024;
+  constexpr int ND = NW + 1;
+  constexpr int WR = 4;  // the tail takes a wave's rows in fours
+  static_assert(R <= RPI && R <= WR && (NS - 1) * ND <= 63, "stage");
+  __shared__ __attribute__((aligned(1024))) uint8_t L0[STAGE], L1[STAGE], L2[STAGE], L3[STAGE];
+  __shared__ float lg[W * WR][kRouterMaxE + 1];
+  // (LDS pointers throughout, so that the compiler ties each read to its
+  // stage and waits for none of the other stages' DMA)
+  auto ST = [&](int i) -> lds_u8* {
+    return i == 0 ? (lds_u8*)L0 : i == 1 ? (lds_u8*)L1 : i == 2 ? (lds_u8*)L2 : (lds_u8*)L3;
+  };
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int E = a.E;
+  const int64_t t0 = (int64_t)blockIdx.x * W * R + wave * R;  // this wave's first row
+  const int nch = (int)(a.H / 64);
+
+  // DMA sources: W k-rows 4 (NW w + q) + lane / 16 at columns 4 (lane % 16)
+  // (clamped to E - 4: the pad columns are never used); x row lane / (64 /
+  // RPI), clamped to the wave's rows and to T
+  uint32_t vw[NW];
+#pragma unroll
+  for (int q = 0; q < NW; ++q)
+    vw[q] = (uint32_t)((4 * (NW * wave + q) + (lane >> 4)) * E + min(4 * (lane & 15), E - 4)) * 4;
+  const int64_t t1 = t0 < a.T ? t0 : a.T - 1;
+  const int64_t tx = t0 + min(lane / (64 / RPI), R - 1);
+  const uint32_t vx =
+      (uint32_t)(((tx < a.T ? tx : a.T - 1) - t1) * a.x_rs * XE + lane % (64 / RPI) * 16);
+  const char* xb = (const char*)a.x + t1 * a.x_rs * XE;
+  // requests chunk i (past the last: nothing) into stage s
+  auto issue = [&](lds_u8* s, int i) __attribute__((always_inline)) {
+    const bool live = i < nch;
+    const int64_t ic = live ? i : 0;
+    const __amdgpu_buffer_rsrc_t rx = router_rsrc(xb + ic * (64 * XE), live ? 0x7fffffffu : 0u);
+    const __amdgpu_buffer_rsrc_t rw = router_rsrc(a.w + ic * 64 * E, live ? 64 * E * 4 : 0);
+    router_dma(rx, vx, s + (16384 + wave * 1024));
+#pragma unroll
+    for (int q = 0; q < NW; ++q) router_dma(rw, vw[q], s + (wave * NW + q) * 1024);
+  };
+  int w_off = lane * 4, x_off = 16384 + wave * 1024;
+  asm("" : "+v"(w_off));
+  asm("" : "+v"(x_off));
+
+  // a quarter chunk: 16 k-rows of W and of each row of x (every lane reads
+  // the same x, an LDS broadcast)
+  constexpr int XQ = 16 * XE / 16;  // 16-byte reads of x per quarter
+  float wv[2][16], acc[R];
+  u32x4_t xv[2][R][XQ];
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+  auto read = [&](lds_u8* s, int g, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int q = 0; q < XQ; ++q)
+        xv[slot][r][q] = *(const lds_u32x4*)(s + (x_off + (r * 64 + g * 16) * XE + q * 16));
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      wv[slot][i] = *(const lds_f32*)(s + (w_off + (g * 16 + i) * 256));
+  };
+  // (x as f32 first, so that no multiply-add waits for its conversion)
+  auto fmas = [&](int slot) __attribute__((always_inline)) {
+    float x[R][16];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if constexpr (XBF16) {
+          const uint32_t d = xv[slot][r][i / 8][(i / 2) % 4];
+          x[r][i] = vm::as_f(i & 1 ? d & 0xffff0000u : d << 16);
+        } else {
+          x[r][i] = vm::as_f(xv[slot][r][i / 4][i % 4]);
+        }
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[r] = fmaf(x[r][i], wv[slot][i], acc[r]);
+  };
+  auto barrier = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto landed = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(router_wait((NS - 2) * ND));
+    barrier();
+  };
+  // chunk i in stage j, its first quarter in slot 0: each quarter's
+  // multiply-adds run behind the next quarter's reads; before the last one
+  // chunk i + 1 has landed and every wave has read chunk i, so the barrier
+  // frees its stage
+  auto step = [&](int j, int i) __attribute__((always_inline)) {
+    lds_u8* s = ST(j);
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+      read(s, g + 1, (g + 1) & 1);
+      __builtin_amdgcn_sched_barrier(0);
+      fmas(g & 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    landed();
+    read(ST((j + 1) % NS), 0, 0);  // (past the last chunk: never used)
+    issue(s, i + NS);
+    __builtin_amdgcn_sched_barrier(0);
+    fmas(1);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i) issue(ST(i), i);
+  landed();
+  read(ST(0), 0, 0);
+  issue(ST(NS - 1), NS - 1);
+  // whole turns of the ring, then the rest (an exit inside the turn would
+  // make the compiler wait for every DMA at the loop's head)
+  int i = 0;
+  for (; i + NS <= nch; i += NS) {
+#pragma unroll
+    for (int j = 0; j < NS; ++j) step(j, i + j);
+  }
+  if (i < nch) {
+    step(0, i);
+    if (i + 1 < nch) {
+      step(1, i + 1);
+      if (i + 2 < nch) step(2, i + 2);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(router_wait(0));
+
+  // lane l holds column l of the wave's rows: the logits (with the bias) go
+  // to the rows' LDS scratch, and 16 lanes read each row's columns back, four
+  // rows a time (with R < 4 the spare lanes run along on zeros)
+  const float bias = a.b[lane < E ? lane : 0];
+#pragma unroll
+  for (int r = 0; r < WR; ++r) lg[WR * wave + r][lane] = r < R ? acc[r < R ? r : 0] + bias : 0.0f;
+  __syncthreads();
+  const int c4 = (lane & 15) * 4;
+  const int r = lane >> 4;
+  float y[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) y[j] = lg[WR * wave + r][c4 + j];
+  router_tail<16, 4>(a, y, c4, r < R ? t0 + r : a.T, lg[WR * wave + r]);
 }
 
 template <bool XBF16>
@@ -403,6 +593,30 @@ bool moe_router_ok(const RouterArgs& a) {
 
 void launch_moe_router(const RouterArgs& a, hipStream_t stream) {
   if (!moe_router_ok(a)) fail(REW_MI355X_ERR_INVALID, "internal: router launch outside its limits");
+  // The row form up to 2048 tokens; us for H 2048, E 64, bf16, against the
+  // matrix-core form: 40 tokens 26.9 / 44.0, 512 29.6 / 45, 1024 32.0 / 45.6,
+  // 2048 41.7 / 46.1; more rows per wave no longer gained (four, with x as
+  // DPP operands, at 4096 tokens 45.0 / 47.3, eight at 8192 72.6 / 49.9).
+  // H 192, E 8, 40 tokens: 11.8 / 14.8 (of the narrow form).  Its offsets
+  // from a wave's first row are 32-bit.
+  if (a.T <= 2048 && a.x_rs >= 0 && a.x_rs < (1 << 24)) {
+    auto grid = [&](int rows) { return dim3((unsigned)((a.T + rows - 1) / rows)); };
+#define REW_ROUTER_ROWS(R, W)                                                                    \
+  do {                                                                                           \
+    if (a.x_bf16)                                                                                \
+      hipLaunchKernelGGL((moe_router_row_kernel<true, R, W>), grid(R * W), dim3(64 * W), 0,      \
+                         stream, a);                                                             \
+    else                                                                                         \
+      hipLaunchKernelGGL((moe_router_row_kernel<false, R, W>), grid(R * W), dim3(64 * W), 0,     \
+                         stream, a);                                                             \
+  } while (0)
+    if (a.T <= 512) REW_ROUTER_ROWS(1, 1);
+    else if (a.T <= 1024) REW_ROUTER_ROWS(1, 4);
+    else REW_ROUTER_ROWS(2, 4);
+#undef REW_ROUTER_ROWS
+    REW_HIP(hipGetLastError());
+    return;
+  }
   if (a.H % 128 == 0) {
     const unsigned blocks = (unsigned)((a.T + 31) / 32);
     if (a.x_bf16)

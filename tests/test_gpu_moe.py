@@ -512,3 +512,15 @@ def test_router_one_launch(gpu, T, H, E_, k, bf16):
         np.testing.assert_array_equal(got[1], ref[1])
         np.testing.assert_array_equal(got[0].view(np.uint32), ref[0].view(np.uint32))
         assert np.all(np.isnan(got[0][3]))
+
+
+@pytest.mark.parametrize("T,H,E_,k,bf16", [(4, 64, 4, 1, True), (6, 128, 64, 16, False),
+                                           (512, 192, 12, 6, True), (513, 256, 64, 6, True),
+                                           (1023, 320, 20, 2, False), (1025, 448, 64, 6, True),
+                                           (2047, 64, 36, 3, False), (2049, 64, 8, 2, True)])
+def test_router_row_form(gpu, T, H, E_, k, bf16):
+    """The router at the edges of the forms that give a wave one or two rows:
+    one chunk of 64 k, fewer chunks than the ring has stages and more, whole
+    turns and remainders, ragged last workgroups, few and all columns."""
+    test_router_one_launch(gpu, T, H, E_, k, bf16)
+
