@@ -180,15 +180,25 @@ __device__ __forceinline__ void tile_order(int64_t bid, int64_t tiles_m, int64_t
 // global_load_lds from per-lane 64-bit addresses (A still through its
 // descriptor): a few VALU instructions per B DMA more than one descriptor,
 // far fewer than the K-tail path.
-template <bool B_KC, bool DUAL, bool GROUP, bool BUF, bool FAR = false>
-__global__ void __launch_bounds__(256, 1) gemm_lds_kernel(GemmSegs gs, GroupArgs ga) {
+// LOW (GROUP and BUF, N-contiguous B): no group has more than
+// kSmallGroupRows rows (a decode step's routing), so only the 64-row body
+// runs.  Its A stages are a quarter as tall, the LDS comes to 80 KiB and two
+// workgroups share a CU: the weight stream is what bounds such a launch, and
+// twice the bytes are in flight while one tile's prologue or epilogue runs.
+// 40 tokens over 64 + 2 experts of 2048 x 1408, the whole block: 277.7 ->
+// 271.3 us (on boxes where one earlier build took 296.1 and 294.6).  Above
+// kSmallGroupRows tokens a group may need 256-row tiles.
+template <bool B_KC, bool DUAL, bool GROUP, bool BUF, bool FAR = false, bool LOW = false>
+__global__ void __launch_bounds__(256, LOW ? 2 : 1) gemm_lds_kernel(GemmSegs gs, GroupArgs ga) {
+  static_assert(!LOW || (GROUP && BUF && !B_KC), "64-row tiles: grouped buffer path");
+  constexpr int PAIR = LOW ? kSmallTileM * 128 : STAGE;  // an A pair stage
   // LDS, 128 KiB.  K-tail path: four 32 KiB stages, each the A and B halves
   // of one k-tile.  BUF path: two 32 KiB A stages, each a k-tile pair (256
   // rows x 128 bytes, so every A row of a pair is one whole cache line), and
   // four 16 KiB B stages.  Each region is its own __shared__ array so the
   // compiler sees that a DMA into one cannot alias fragment reads of another.
-  __shared__ __attribute__((aligned(1024))) uint8_t L0[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t L1[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t L0[PAIR];
+  __shared__ __attribute__((aligned(1024))) uint8_t L1[PAIR];
   __shared__ __attribute__((aligned(1024))) uint8_t L2[BUF ? B_BYTES : STAGE];
   __shared__ __attribute__((aligned(1024))) uint8_t L3[BUF ? B_BYTES : STAGE];
   __shared__ __attribute__((aligned(1024))) uint8_t L4[BUF ? B_BYTES : 16];
@@ -202,7 +212,8 @@ __global__ void __launch_bounds__(256, 1) gemm_lds_kernel(GemmSegs gs, GroupArgs
   };
   // 16 KiB block blk (rows 32 blk .. 32 blk + 31) of the epilogue's C tile
   auto CB = [&](int blk) -> uint8_t* {
-    if constexpr (BUF) return blk < 4 ? AS(blk >> 1) + (blk & 1) * B_BYTES : BS(blk - 4);
+    if constexpr (LOW) return BS(blk);  // (two blocks)
+    else if constexpr (BUF) return blk < 4 ? AS(blk >> 1) + (blk & 1) * B_BYTES : BS(blk - 4);
     else return S(blk >> 1) + (blk & 1) * B_BYTES;
   };
   const int tid = threadIdx.x, lane = tid & 63;
@@ -918,12 +929,12 @@ __global__ void __launch_bounds__(256, 1) gemm_lds_kernel(GemmSegs gs, GroupArgs
   };  // run
 
   if constexpr (GROUP && BUF && !B_KC) {
-    if (small) {  // (uniform)
+    if (LOW || small) {  // (uniform)
       run(IntK<1>{});
       return;
     }
   }
-  run(IntK<0>{});
+  if constexpr (!LOW) run(IntK<0>{});
 }
 
 // Conditions of the gemm_lds kernels: bf16 in / out, K-contiguous A with
@@ -982,6 +993,19 @@ static void launch_segs(const GemmSegs& gs, const GroupArgs* ga, bool bkc, int b
   const GroupArgs none{};
   const GroupArgs& G = ga ? *ga : none;
   const dim3 grid((unsigned)tiles), block(256);
+  if (ga && buf && !bkc && ga->max_rows >= 0 && ga->max_rows <= kSmallGroupRows) {
+    if (dual && buf == 2)
+      hipLaunchKernelGGL((gemm_lds_kernel<false, true, true, true, true, true>), grid, block, 0,
+                         stream, gs, G);
+    else if (dual)
+      hipLaunchKernelGGL((gemm_lds_kernel<false, true, true, true, false, true>), grid, block, 0,
+                         stream, gs, G);
+    else
+      hipLaunchKernelGGL((gemm_lds_kernel<false, false, true, true, false, true>), grid, block, 0,
+                         stream, gs, G);
+    REW_HIP(hipGetLastError());
+    return;
+  }
 #define REW_LDS_LAUNCH(BKC, DU, GR)                                                          \
   do {                                                                                      \
     if (DU && buf == 2)                                                                     \

@@ -145,6 +145,8 @@ struct GroupArgs {
   // host side: the largest |b2[i] - b[i]| in bytes (the dual B operands
   // share one buffer descriptor when it is small), -1 when not known
   int64_t dual_span = -1;
+  // host side: a bound on every group's rows, -1 when not known
+  int64_t max_rows = -1;
 };
 // Whether launch_gemm_grouped can run g (dtype, layout, epilogue, 32-bit
 // buffer extents).

@@ -244,6 +244,7 @@ void run_routed_ffn(Ctx* c, const RoutedFfn& a, void* scratch) {
   ga.n_groups = groups;
   // (a group of r rows takes at most r / 256 + 2 tiles, group_tiles)
   ga.max_mtiles = (R + 255) / 256 + 2 * n + (int64_t)ns * group_tiles(a.T);
+  ga.max_rows = a.T;  // (a token counts once in a group)
   ga.rows = ra.perm;
   ga.b = tables;
   ga.b2 = tables + groups;

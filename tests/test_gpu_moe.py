@@ -136,6 +136,24 @@ def test_moe_sparse_equals_dense_op_by_op(gpu, oracle):
     np.testing.assert_array_equal(sparse, dense)
 
 
+@pytest.mark.parametrize("T,H,I,n_shared", [(1, 256, 128, 1), (40, 128, 192, 2),
+                                            (64, 192, 320, 1), (65, 256, 136, 2),
+                                            (128, 64, 64, 0), (129, 256, 192, 1)])
+def test_moe_few_tokens(gpu, oracle, T, H, I, n_shared):
+    """Up to 128 tokens every group takes 64-row tiles, by a kernel of their
+    own; each output keeps its MFMA sequence, so the values equal the dense
+    op-by-op ones (129 tokens and I 136 take the other kernels)."""
+    moe, host = build_moe(oracle, T, H, I, 8, 2, n_shared, 0x5EED0505 + T)
+    xt = E.fromHost(host["x"], DType.BFLOAT16)
+    sparse = E.toHostF32(moe.forward(xt))
+    E.setMode(E.MODE_OP_BY_OP)
+    try:
+        dense = E.toHostF32(moe.forward(xt))
+    finally:
+        E.setMode(E.MODE_DEFERRED)
+    np.testing.assert_array_equal(sparse, dense)
+
+
 def small_and_large_groups(oracle):
     """Groups of more than 128 rows (256-row tiles, ragged last ones), of
     65-128 rows (two 64-row tiles) and of at most 64 rows (one) in the same
