@@ -522,9 +522,11 @@ def run_chain(args, steps=None, warmup=None):
         if name.startswith("ew_"):  # the relu chain, or the [8192] divide of reduceMean
             return groups["relu_chain"] if name.startswith(f"ew_fused{{{R * Cn}x") else 3 * R * 4
         if name.startswith("reduce"):
-            # one read of x; one [R] output per op, plus reduceMean's quotient
+            # one read of x (and the chain's store, where the pass keeps it); one
+            # [R] output per op, plus reduceMean's quotient
             ops = int(name.split("ops")[0].rsplit(",", 1)[1]) if "ops" in name else 1
-            return nbytes + R * 4 * (ops + (1 if ",mean" in name else 0))
+            full = groups["relu_chain"] if ",kept" in name else nbytes
+            return full + R * 4 * (ops + (1 if ",mean" in name else 0))
         return None
 
     syms = by_symbol(prof, bytes_of)

@@ -247,6 +247,8 @@ std::string signature(const vm::Program& P, const vm::Space& S, int kind, int V,
     put(&A->n_mean, sizeof A->n_mean);
     put(A->mean_src, sizeof(int) * A->n_mean);
     put(A->mean_div, sizeof(float) * A->n_mean);
+    const bool keep = A->keep != nullptr;
+    put(&keep, sizeof keep);
   }
   return k;
 }
@@ -450,6 +452,7 @@ std::string gen_reduce(const vm::Program& P, const vm::Space& S, const ReduceArg
     << (P.n_leaves ? ", " : "") << "void* out";
   for (int x = 0; x < A.n_extra; ++x) o << ", void* out" << x + 1;
   for (int x = 0; x < A.n_mean; ++x) o << ", void* mean" << x;
+  if (A.keep) o << ", void* keep";
   o << ") {\n";
   put_space(o, S);
   put_leaves(o, P);
@@ -496,7 +499,24 @@ std::string gen_reduce(const vm::Program& P, const vm::Space& S, const ReduceArg
       o << "    const uint32_t lin" << sfx << " = r_out * n_red + r" << sfx << ";\n";
       o << "    int32_t c" << sfx << "[kRank]; delinearize(S, lin" << sfx << ", c" << sfx << ");\n";
     }
-    for (int u = 0; u < kUnroll; ++u) {
+    if (A.keep) {
+      // every load before the first store: a store under its row's bound is
+      // a branch, at which the compiler waits for the loads in flight
+      std::string val[kUnroll];
+      for (int u = 0; u < kUnroll; ++u) {
+        const std::string sfx = "_" + std::to_string(u);
+        put_body(o, P, V, sfx.c_str(), outs, ("lin" + sfx).c_str(), ("c" + sfx).c_str());
+        val[u] = outs[0];
+      }
+      for (int u = 0; u < kUnroll; ++u) {
+        const std::string sfx = "_" + std::to_string(u);
+        o << "    if (ok" << sfx << ") {\n     store_vec<" << V << ">(keep, " << kF32
+          << ", (int64_t)lin" << sfx << ", " << val[u] << ");\n     for (int j = 0; j < " << V
+          << "; ++j) {\n"
+          << accs("      acc@ = red_op_j(%, acc@, " + val[u] + "[j]);\n") << "     }\n    }\n";
+      }
+    }
+    for (int u = 0; u < kUnroll && !A.keep; ++u) {
       const std::string sfx = "_" + std::to_string(u);
       put_body(o, P, V, sfx.c_str(), outs, ("lin" + sfx).c_str(), ("c" + sfx).c_str());
       o << "    if (ok" << sfx << ") for (int j = 0; j < " << V << "; ++j) {\n"
@@ -528,8 +548,8 @@ std::string gen_reduce(const vm::Program& P, const vm::Space& S, const ReduceArg
 
 bool launch(JitFn* f, const vm::Program& P, const ReduceArgs* A, bool outs, int64_t blocks,
             hipStream_t stream) {
-  void* args[vm::kMaxLeaves + vm::kMaxOuts + 4];
-  const void* ptrs[vm::kMaxLeaves + vm::kMaxOuts + 4];
+  void* args[vm::kMaxLeaves + vm::kMaxOuts + 7];  // (a reduction has up to 7)
+  const void* ptrs[vm::kMaxLeaves + vm::kMaxOuts + 7];
   int n = 0;
   for (int i = 0; i < P.n_leaves; ++i) ptrs[n++] = P.leaf[i].ptr;
   if (outs)
@@ -538,6 +558,7 @@ bool launch(JitFn* f, const vm::Program& P, const ReduceArgs* A, bool outs, int6
     ptrs[n++] = A->out;
     for (int x = 0; x < A->n_extra; ++x) ptrs[n++] = A->extra_out[x];
     for (int x = 0; x < A->n_mean; ++x) ptrs[n++] = A->mean_out[x];
+    if (A->keep) ptrs[n++] = A->keep;
   }
   for (int i = 0; i < n; ++i) args[i] = (void*)&ptrs[i];
   REW_HIP(hipModuleLaunchKernel(f->fn, (unsigned)blocks, 1, 1, 256, 1, 1, 0, stream, args,

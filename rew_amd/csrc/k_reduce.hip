@@ -106,6 +106,18 @@ void launch_reduce(const vm::Program& P, const vm::Space& S,
                    const ReduceArgs& A, bool vec, hipStream_t stream) {
   if (A.n_out == 0) return;
   if (jit_launch_reduce(P, S, A, vec, stream)) return;
+  if (A.keep) {
+    // the interpreter stores the values in a pass of their own
+    vm::Program E = P;
+    E.out[0].ptr = A.keep;
+    E.out[0].dtype = REW_DT_FLOAT32;
+    E.out[0].off = 0;
+    launch_ew(E, S, vec, stream);
+    ReduceArgs plain = A;
+    plain.keep = nullptr;
+    launch_reduce(P, S, plain, vec, stream);
+    return;
+  }
   if (A.n_mean > 0) {
     // the interpreter stores the sums, then divides them
     ReduceArgs plain = A;

@@ -52,6 +52,9 @@ struct ReduceArgs {
   int mean_src[2] = {0, 0};
   float mean_div[2] = {1.0f, 1.0f};
   void* mean_out[2] = {nullptr, nullptr};
+  // the reduced values themselves (f32, in the space's linear order), where
+  // something else reads them too; rows of at least 128 values
+  void* keep = nullptr;
 };
 // Space = [kept..., reduced...]; program output 0 names the value register.
 void launch_reduce(const vm::Program& P, const vm::Space& S,

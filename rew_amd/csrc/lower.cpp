@@ -332,6 +332,9 @@ struct Lower {
   // (reduceMean's reduceSum next to a reduceSum of the same tensor) aliases
   // the first result
   std::map<std::tuple<Tensor*, int, std::vector<int64_t>, int>, Tensor*> reduce_done;
+  Tensor* keep_src = nullptr;              // the next reduction stores its source too
+  std::unordered_set<Tensor*> keep_failed; // sources whose program did not fit there
+  Node* keeping_reduction(Tensor* t);
   // dense copies made by emit_permuted_copy and not yet freed: released
   // (stream-ordered) when their consumer is enqueued or at the end of the flush
   std::unordered_set<Tensor*> temps;
@@ -1009,6 +1012,11 @@ void Lower::ensure_mat(Tensor* t) {
         return;
       }
     }
+    if (Node* r = keeping_reduction(t)) {
+      keep_src = t;
+      emit_reduce(r);
+      if (t->st) return;
+    }
     emit_ew_root(t);
     return;
   }
@@ -1116,9 +1124,45 @@ void Lower::emit_anchor(Node* n) {
   }
 }
 
+// A reduction over the trailing axes of the elementwise tensor t, about to
+// be materialized, that can store t on its way: t is then not read back.  A
+// wave takes a row, so the rows have to fill the SIMDs (1024 of them), and
+// 16-byte vectors have to fit them.  8192 x 4096: the chain, its sum, mean
+// and max, softmax and rmsNorm of its input 164.7 -> 144.0 us, the sum's own
+// read of 134 MB and a launch gone.
+Node* Lower::keeping_reduction(Tensor* t) {
+  if (t->dt != kF32 || !is_ew(t->prod->kind) || keep_failed.count(t)) return nullptr;
+  auto ci = cons.find(t);  // (empty where every op is its own launch)
+  if (ci == cons.end()) return nullptr;
+  for (Node* r : ci->second) {
+    if (r->kind != K_REDUCE || r->in[0] != t || r->l0.empty() || r->out[0]->st ||
+        !r->out[0]->plan_mat)
+      continue;
+    const Shape& X = t->shape;
+    std::vector<bool> red(X.rank, false);
+    for (auto d : r->l0) red[d] = true;
+    int64_t n_out = 1, n_red = 1;
+    bool trailing = true;
+    for (int i = 0; i < X.rank; ++i) {
+      trailing = trailing && (red[i] || n_red == 1);
+      if (red[i]) n_red *= X.d[i];
+      else n_out *= X.d[i];
+      if (red[i] && X.d[i] == 1) trailing = false;
+    }
+    if (trailing && n_red >= 128 && n_red % kVec == 0 && n_out >= 1024) return r;
+  }
+  return nullptr;
+}
+
 void Lower::emit_reduce(Node* n) {
   Tensor* x = n->in[0];
   Tensor* out = n->out[0];
+  bool keep = keep_src == x;
+  keep_src = nullptr;
+  if (!keep && x->plan_mat && !x->st && x->prod && is_ew(x->prod->kind)) {
+    ensure_mat(x);
+    if (out->st) return;  // (stored by the reduction that kept x)
+  }
   const auto key = std::make_tuple(x, n->sub, n->l0, out->dt);
   auto done = reduce_done.find(key);
   if (done != reduce_done.end() && done->second->st && done->second->shape == out->shape) {
@@ -1147,11 +1191,14 @@ void Lower::emit_reduce(Node* n) {
   for (int attempt = 0; attempt < 2; ++attempt) {
     Gen g(*this, space);
     try {
-      int v = g.gen(x, m);
+      int v = keep ? g.gen_node(x->prod, x, m) : g.gen(x, m);
       std::vector<int64_t> dims;
       // collapse; keep the kept/reduced boundary
       Space S = finish_space(g.P, space, n_kept, &dims);
       check_bounds(g.P, g.leaf_t, dims);
+      const bool vec = n_red > 0 && (dims.back() % kVec) == 0 &&
+                       (n_red % kVec) == 0 && space.d[X.rank - 1] != 1;
+      if (keep && !vec) throw GenFail{};
       std::vector<int> phys;
       alloc_regs(g.P, {v}, &phys);
       g.P.n_outs = 1;
@@ -1208,15 +1255,17 @@ void Lower::emit_reduce(Node* n) {
           }
         }
       }
-      const bool vec = n_red > 0 && (dims.back() % kVec) == 0 &&
-                       (n_red % kVec) == 0 && space.d[X.rank - 1] != 1;
+      if (keep) {
+        tensor_alloc(x);
+        A.keep = x->data();
+      }
       set_leaf_modes(g.P, S, vec);
       Launch L{ReduceL{g.P, S, A, vec}};
       if (c->profiling)
         L.name = "reduce{" + std::to_string(n_out) + "x" + std::to_string(n_red) + "x" +
                  std::to_string(g.P.n_ins) +
                  (sib.empty() ? "" : "," + std::to_string(1 + sib.size()) + "ops") +
-                 (A.n_mean ? ",mean" : "") + "}";
+                 (A.n_mean ? ",mean" : "") + (keep ? ",kept" : "") + "}";
       L.fused = g.P.n_ins > 1 || !sib.empty();
       run_launch(c, std::move(L));
       reduce_done[key] = out;
@@ -1224,6 +1273,10 @@ void Lower::emit_reduce(Node* n) {
       return;
     } catch (GenFail&) {
       tensor_drop_storage(out);
+      if (keep) {
+        keep = false;
+        keep_failed.insert(x);
+      }
       x->plan_mat = true;
       ensure_mat(x);
     }

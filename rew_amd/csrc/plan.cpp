@@ -46,6 +46,7 @@ struct PtrVisit {
     field(f, l.A.out);
     for (int i = 0; i < l.A.n_extra; ++i) field(f, l.A.extra_out[i]);
     for (int i = 0; i < l.A.n_mean; ++i) field(f, l.A.mean_out[i]);
+    if (l.A.keep) field(f, l.A.keep);
   }
   void operator()(GemmL& l) {
     for (GemmArgs& g : l.g) {

@@ -644,3 +644,59 @@ def test_embedding_lookup_rmsnorm_one_pass(gpu, oracle, ids_dt):
     np.testing.assert_array_equal(E.bf16_bits_to_f32(got[1]).reshape(T, H), rows)
     want = oracle.rmsnorm_rows(rows, g, 1e-5)
     bf16_close(E.bf16_bits_to_f32(got[0]).reshape(T, H), want, 1e-2)
+
+
+KEPT_CHILD = r"""
+import json, sys
+import numpy as np
+sys.path.insert(0, sys.argv[1])
+from rew_amd import eager as E, nn, ops as O
+E.installEagerBackend(E.mi355x(0))
+for shape, axes, kept in json.loads(sys.argv[2]):
+    print(shape, flush=True)
+    rng = np.random.default_rng(sum(shape))
+    x = rng.standard_normal(shape, np.float32)
+    x[0, ..., 3] = np.inf
+    x[1, ..., 5] = np.nan
+    x[-1] = -0.0
+    b = rng.standard_normal(shape[-1:], np.float32)
+    def fn():
+        xt = E.fromHost(x)
+        y = nn.relu(O.add(xt, O.broadcastTo(E.fromHost(b), shape, [len(shape) - 1])))
+        outs = [y, O.reduceSum(y, axes), O.reduceMean(y, axes), O.reduceMax(y, axes)]
+        E.flush()
+        return outs
+    E.profileBegin()
+    outs = fn()
+    names = [n for n, _, _ in E.profileEnd()]
+    assert any(",kept" in n for n in names) == kept, names
+    got = [E.toHost(t) for t in outs]
+    again = [E.toHost(t) for t in fn()]  # (the recorded plan)
+    E.setMode(E.MODE_OP_BY_OP)
+    want = [E.toHost(t) for t in fn()]
+    E.setMode(E.MODE_DEFERRED)
+    for g, a, w in zip(got, again, want):
+        for v in (g, a):
+            np.testing.assert_array_equal(v, w)
+            np.testing.assert_array_equal(np.signbit(v[v == v]), np.signbit(w[w == w]))
+"""
+
+
+@pytest.mark.parametrize("compiled", ["1", "0"])
+def test_reduction_stores_the_chain_it_reads(gpu, compiled):
+    """An elementwise chain that is both returned and reduced over its
+    trailing axes is one pass from 1024 rows of at least 128 values on (a
+    multiple of 4): the same bits as op by op, compiled or interpreted.  The
+    last shapes keep the chain's own pass."""
+    import json
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    cases = [((1024, 128), [1], True), ((1030, 132), [1], True), ((2, 600, 1000), [2], True),
+             ((1025, 4100), [1], True), ((1100, 2, 64), [1, 2], True), ((1023, 256), [1], False),
+             ((1024, 130), [1], False), ((1024, 124), [1], False), ((256, 1024), [0], False)]
+    r = subprocess.run([sys.executable, "-c", KEPT_CHILD, str(Path(__file__).resolve().parents[1]),
+                        json.dumps(cases)], env=dict(os.environ, REW_MI355X_JIT=compiled),
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, (r.stdout[-500:], r.stderr[-3000:])
