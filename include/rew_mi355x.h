@@ -250,7 +250,10 @@ int rew_mi355x_profile_entry(rew_mi355x_ctx* ctx, int index, char* name,
                              int name_cap, int64_t* launches, double* total_ms);
 
 /* Native stream of the context (a hipStream_t), for callers that record
- * their own events around the backend's work. */
+ * their own events around the backend's work.  Split products and decode
+ * attention keep partial results in one array per GPU, ordered by this
+ * stream: launches captured from it must not be replayed on another stream
+ * while it has work. */
 int rew_mi355x_stream(rew_mi355x_ctx* ctx, void** out_stream);
 
 /* ---- routed mixture-of-experts FFN over caller-owned device rows ---------

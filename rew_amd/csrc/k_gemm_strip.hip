@@ -28,8 +28,8 @@
 // Measured (weights out of cache; K x N, before -> after): 14336 x 4096 at 8,
 // 64, 300 and 1000 rows 443 -> 28, 449 -> 33, 451 -> 60, 460 -> 150 us;
 // 4096 x 4096 at 8, 300, 1000 rows 120 -> 14, 131 -> 25, 131 -> 46 us; SwiGLU
-// 4096 x 14336 at 8 rows 95 -> 52 us (4.5 TB/s of weights; a copy reaches
-// 4.7 TB/s on the card).
+// 4096 x 14336 at 8 rows 95 -> 52 us (4.5 TB/s of weights; a 1 GiB
+// copy reaches 6.2 TB/s).
 #include <cstdlib>
 #include <cstring>
 
