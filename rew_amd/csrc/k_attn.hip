@@ -116,16 +116,41 @@ __device__ __forceinline__ void dma16(const void* src, uint16_t* lds) {
   __builtin_amdgcn_global_load_lds(src, (lds_void*)lds, 16, 0, 0);
 }
 
-// Buffer descriptor over `base` with no range limit (callers keep every
-// offset inside the tensor); the base is wave-uniform and readfirstlane
-// says so, which keeps the descriptor in SGPRs.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t fa_rsrc(const void* base) {
+// Buffer descriptor over `bytes` bytes at `base`; a read past them returns
+// zeros and touches no memory.  Both are wave-uniform and readfirstlane says
+// so, which keeps the descriptor in SGPRs.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t fa_rsrc(const void* base,
+                                                          uint32_t bytes = 0x7fffffff) {
   const uint64_t a = (uint64_t)(uintptr_t)base;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
   void* p = (void*)(uintptr_t)(((uint64_t)hi << 32) | lo);
-  return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, 0x7fffffff, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, (int)__builtin_amdgcn_readfirstlane(bytes),
+                                           0x00020000);
 }
+// Walks key rows of D bf16 values, `stride` (>= 0) apart, a tile at a time
+// from row k0 of `rows` to the next one `step` rows on (additions on the
+// scalar ALU only: a multiplication per tile cost a decode step up to 10 %).
+// The rows past the last one read as zeros, so a ragged last tile takes the
+// same DMA as the others: its missing K rows score 0 (and are dropped before
+// the softmax), its missing V rows add 0 times 0.  The advance is in the
+// descriptor's base, where the range check sees it.
+struct FaRows {
+  const uint16_t* p;
+  int64_t step;
+  int left;  // bytes from p to the end of the last row
+  __device__ __forceinline__ FaRows(const uint16_t* base, int k0, int rows, int64_t stride, int D,
+                                    int step_rows)
+      : p(base + k0 * stride), step(step_rows * stride),
+        left((int)(((rows - 1 - k0) * stride + D) * 2)) {}
+  // the descriptor of this tile (none of it unless live), and on to the next
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t next(bool live) {
+    const __amdgpu_buffer_rsrc_t r = fa_rsrc(p, live ? (uint32_t)left : 0u);
+    p += step;
+    left -= (int)step * 2;
+    return r;
+  }
+};
 // 16 bytes per lane from base + voff + soff into LDS (buffer_load ... lds):
 // the per-lane offset is fixed, the tile advance is the scalar `soff`.
 __device__ __forceinline__ void dma16_buf(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
@@ -145,10 +170,8 @@ __device__ __forceinline__ void dma16_lds(__amdgpu_buffer_rsrc_t r, uint32_t vof
 //   1 diagonal  a whole tile under an ordered mask that adds 0 where
 //               visible, scale > 0: t = fma(x, scale log2 e, visible ? 0 :
 //               mask_false log2 e), visibility from one per-lane threshold;
-//   2 general   anything else: t = (x * scale + mask) log2 e, -inf past Sk
-//               and below jlo, from which a ragged last tile that was moved
-//               back to end at Sk counts its keys;
-//   4 tail      such a tile without a mask, scale > 0: -inf below jlo.
+//   2 general   anything else: t = (x * scale + mask) log2 e, -inf past Sk;
+//   4 tail      a ragged last tile without a mask, scale > 0: -inf past Sk.
 // The plain tiles of queries [q0, q_last] form one range of key tiles
 // [lo, hi), found once per wave group instead of per tile.
 struct FaKinds {
@@ -218,7 +241,7 @@ __device__ __forceinline__ float fa_round_max(f32x16_t (&sacc)[2]) {
 // below the diagonal, FA_GENERAL).
 enum { FA_PLAIN = 0, FA_DIAG_UP = 1, FA_GENERAL = 2, FA_DIAG_DOWN = 3, FA_TAIL = 4 };
 template <int DT, int KIND>
-__device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int jlo, int qi, int g,
+__device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int qi, int g,
                                                 float sl2, f32x16_t (&sacc_in)[2],
                                                 float mr, uint32_t (&pk)[2][8], float& m_run,
                                                 float& l_run, float& alpha_out) {
@@ -230,12 +253,12 @@ __device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int 
   } else if constexpr (KIND == FA_DIAG_UP || KIND == FA_DIAG_DOWN || KIND == FA_TAIL) {
     // key j = k0 + off (off = kb 32 + (e / 4) 8 + g 4 + e % 4) is visible
     // iff j - qi >= lo (LE, LT) or j - qi <= -lo (GE, GT)
-    // (tail: j >= jlo, and -inf below)
-    constexpr bool kUp = KIND != FA_DIAG_DOWN;
+    // (tail: j < Sk, and -inf past it)
+    constexpr bool kUp = KIND == FA_DIAG_UP;
     const float mf2 = KIND == FA_TAIL ? -INFINITY : a.mask_false * kLog2e;
     const int lo = (a.cmp == vm::CMP_LT || a.cmp == vm::CMP_GT) ? 1 : 0;
     const int base = k0 - qi + g * 4;
-    const int thr = KIND == FA_TAIL ? jlo - k0 - g * 4 : kUp ? lo - base : -lo - base;
+    const int thr = KIND == FA_TAIL ? a.Sk - 1 - k0 - g * 4 : kUp ? lo - base : -lo - base;
     float m0 = -INFINITY, m1 = -INFINITY;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -264,8 +287,8 @@ __device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int 
           x0 += fa_visible(a.cmp, qi, j0) ? a.mask_true : a.mask_false;
           x1 += fa_visible(a.cmp, qi, j0 + 1) ? a.mask_true : a.mask_false;
         }
-        x0 = j0 >= jlo && j0 < a.Sk ? x0 * kLog2e : -INFINITY;
-        x1 = j0 + 1 >= jlo && j0 + 1 < a.Sk ? x1 * kLog2e : -INFINITY;
+        x0 = j0 < a.Sk ? x0 * kLog2e : -INFINITY;
+        x1 = j0 + 1 < a.Sk ? x1 * kLog2e : -INFINITY;
         t[kb][e] = x0;
         t[kb][e + 1] = x1;
         m0 = fmaxf(m0, fmaxf(x0, x1));
@@ -335,19 +358,19 @@ __device__ __forceinline__ float fa_row_sum(const uint32_t (&pk)[2][8]) {
 
 // The softmax step of the tile's kind (fa_kind), then the rescale of O.
 template <int DT>
-__device__ __forceinline__ void fa_softmax_any(int kind, const FlashArgs& a, int k0, int jlo,
-                                               int qi, int g, float sl2, f32x16_t (&sacc)[2],
+__device__ __forceinline__ void fa_softmax_any(int kind, const FlashArgs& a, int k0, int qi,
+                                               int g, float sl2, f32x16_t (&sacc)[2],
                                                float mr, uint32_t (&pk)[2][8], f32x16_t (&o)[DT],
                                                float& m_run, float& l_run) {
   float alpha;
   if (kind == FA_PLAIN)
-    fa_softmax_tile<DT, FA_PLAIN>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_PLAIN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   else if (kind == FA_DIAG_UP)
-    fa_softmax_tile<DT, FA_DIAG_UP>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_DIAG_UP>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   else if (kind == FA_DIAG_DOWN)
-    fa_softmax_tile<DT, FA_DIAG_DOWN>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_DIAG_DOWN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   else
-    fa_softmax_tile<DT, FA_GENERAL>(a, k0, jlo, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    fa_softmax_tile<DT, FA_GENERAL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
   fa_rescale<DT>(o, alpha);
 }
 
@@ -363,10 +386,9 @@ __device__ __forceinline__ void block_barrier_fa() {
   asm volatile("" ::: "memory");
 }
 
-// BUF: at least one whole key tile (a ragged last one is moved back to end at
-// Sk and drops the keys it repeats) and every byte offset into K and V below
-// 2^31, so the tiles move by buffer loads with a scalar tile
-// offset (no per-tile address arithmetic on the vector ALU).
+// BUF: every byte offset into K and V is below 2^31, so the tiles move by
+// buffer loads whose descriptor carries the tile advance (no per-tile address
+// arithmetic on the vector ALU) and reads the rows past Sk as zeros.
 // ROUND: scores are rounded to bf16 before the scale (a.round_scores).
 template <int D, bool BUF, bool ROUND>
 __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
@@ -441,10 +463,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
   // ROWS_PER_DMA * (wave * DMA_PER_WAVE + q) + lane / CPR
   const int row_in = lane / CPR, pc = lane % CPR;
   uint32_t vk_off[DMA_PER_WAVE], vv_off[DMA_PER_WAVE];
-  __amdgpu_buffer_rsrc_t rk, rv;
   if constexpr (BUF) {
-    rk = fa_rsrc(K);
-    rv = fa_rsrc(V);
 #pragma unroll
     for (int q = 0; q < DMA_PER_WAVE; ++q) {
       const int r = (wave * DMA_PER_WAVE + q) * ROWS_PER_DMA + row_in;
@@ -452,15 +471,15 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
       vv_off[q] = (uint32_t)((r * a.v_ss + (pc ^ ((4 * (r & 3)) % CPR)) * 8) * 2);
     }
   }
-  auto dma_tile = [&](uint16_t* ks, uint16_t* vs, int kt) {
-    const int k0 = BUF ? min(kt * BKV, a.Sk - BKV) : kt * BKV;
+  FaRows kw(K, kt0 * BKV, a.Sk, a.k_ss, D, BKV), vw(V, kt0 * BKV, a.Sk, a.v_ss, D, BKV);
+  auto dma_tile = [&](uint16_t* ks, uint16_t* vs, int kt) {  // (kt: one after another)
     if constexpr (BUF) {
-      const uint32_t sk = (uint32_t)(k0 * a.k_ss * 2), sv = (uint32_t)(k0 * a.v_ss * 2);
+      const __amdgpu_buffer_rsrc_t rk = kw.next(kt < kt1), rv = vw.next(kt < kt1);
 #pragma unroll
       for (int q = 0; q < DMA_PER_WAVE; ++q) {
         const int blk = wave * DMA_PER_WAVE + q;
-        dma16_buf(rk, vk_off[q], sk, ks + blk * 512);
-        dma16_buf(rv, vv_off[q], sv, vs + blk * 512);
+        dma16_buf(rk, vk_off[q], 0, ks + blk * 512);
+        dma16_buf(rv, vv_off[q], 0, vs + blk * 512);
       }
       return;
     }
@@ -468,7 +487,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
     for (int q = 0; q < DMA_PER_WAVE; ++q) {
       const int blk = wave * DMA_PER_WAVE + q;
       const int r = blk * ROWS_PER_DMA + row_in;
-      int key = k0 + r;
+      int key = kt * BKV + r;
       key = key < a.Sk ? key : a.Sk - 1;  // rows past Sk: an in-range row (masked below)
       const int ck = pc ^ (r % CPR);
       const int cv = pc ^ ((4 * (r & 3)) % CPR);
@@ -506,9 +525,9 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
 
   auto k_tile = [&](const uint16_t* ks, const uint16_t* vs, uint16_t* ks_n, uint16_t* vs_n,
                     int kt) {
-    const bool more = kt + 1 < kt1;
-    // branch-free: on the last tile a spare reload of tile kt0 into the idle stage
-    dma_tile(ks_n, vs_n, more ? kt + 1 : kt0);
+    // branch-free: on the last tile a spare request into the idle stage, of
+    // nothing (BUF) or of tile kt0
+    dma_tile(ks_n, vs_n, BUF || kt + 1 < kt1 ? kt + 1 : kt0);
 
     // S^T tile: 64 keys x 32 queries as two 32x32 accumulators.  The K
     // fragments of k-step t + 2 are read while the MFMAs of step t run (a
@@ -558,8 +577,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(FlashArgs a) {
     const int k0 = kt * BKV;
     uint32_t pk[2][8];  // bf16 probability pairs: [kb][e/2]
     const float mr = fa_round_max<ROUND>(sacc);
-    fa_softmax_any<DT>(fa_kind(kinds, kt), a, BUF ? min(k0, a.Sk - BKV) : k0, k0, qi, g, sl2, sacc,
-                       mr, pk, o, m_run, l_run);
+    fa_softmax_any<DT>(fa_kind(kinds, kt), a, k0, qi, g, sl2, sacc, mr, pk, o, m_run, l_run);
     l_run = __fadd_rn(l_run, fa_row_sum(pk));
 
     // O^T += V^T P^T over 4 k-steps of 16 keys
@@ -845,8 +863,7 @@ __global__ void __launch_bounds__(512, 1) flash_pp_kernel(FlashArgs a) {
   float mr = -INFINITY;  // max of the rounded scores of the last S tile
   auto soft_phase = [&](int m) {
     const int k0 = (kt0 + m) * BKV;
-    fa_softmax_any<DT>(fa_kind(kinds, kt0 + m), a, k0, k0, qi, g, sl2, sacc, mr, pk, o, m_run,
-                       l_run);
+    fa_softmax_any<DT>(fa_kind(kinds, kt0 + m), a, k0, qi, g, sl2, sacc, mr, pk, o, m_run, l_run);
   };
   // the MFMA phase's share of the softmax: the scores' rounding and max,
   // and the row sum of the last probabilities (in the softmax phase instead
@@ -960,8 +977,8 @@ __global__ void __launch_bounds__(512, 1) flash_pp_kernel(FlashArgs a) {
 // What bounds it is the K / V stream: every wave owns its key tiles (64
 // keys, every second one) and two LDS stages for them, 32 KiB of K and V at
 // D = 128, one in flight by DMA while the other is used, so the waves need no
-// barriers and a CU keeps 64 KiB in flight.  A ragged last tile is moved back
-// to end at Sk; past the last tile the DMA goes through a descriptor of
+// barriers and a CU keeps 64 KiB in flight.  The rows past Sk of a ragged last
+// tile read as zeros; past the last tile the DMA goes through a descriptor of
 // zero records and costs nothing.
 //
 // A wave's running max, sum and O (fp32) join the other wave's through LDS;
@@ -1011,15 +1028,8 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
 #pragma unroll
     for (int t = 0; t < NT; ++t) qf[t] = *(const bf16x8_t*)(qp + t * 16 + g * 8);
   }
-  const uint64_t K = (uint64_t)(uintptr_t)((const uint16_t*)a.k + b * a.k_sb + hk * a.k_sh);
-  const uint64_t V = (uint64_t)(uintptr_t)((const uint16_t*)a.v + b * a.v_sb + hk * a.v_sh);
-  auto rsrc = [](uint64_t p, uint32_t bytes) {
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)p);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(p >> 32));
-    return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)(((uint64_t)hi << 32) | lo),
-                                             (short)0, __builtin_amdgcn_readfirstlane((int)bytes),
-                                             0x00020000);
-  };
+  const uint16_t* K = (const uint16_t*)a.k + b * a.k_sb + hk * a.k_sh;
+  const uint16_t* V = (const uint16_t*)a.v + b * a.v_sb + hk * a.v_sh;
   // the layouts of flash_fwd_kernel: chunk pc of key row r holds logical chunk
   // pc ^ (r % CPR) of K and pc ^ (4 (r & 3)) of V
   const int row_in = lane / CPR, pc = lane % CPR;
@@ -1030,16 +1040,14 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
     kv_off[q] = (uint32_t)((r * a.k_ss + (pc ^ (r % CPR)) * 8) * 2);
     vv_off[q] = (uint32_t)((r * a.v_ss + (pc ^ ((4 * (r & 3)) % CPR)) * 8) * 2);
   }
-  auto dma_tile = [&](lds_u16* st, int i) {
-    const uint32_t bytes = i < n ? 0x7fffffffu : 0u;
-    const __amdgpu_buffer_rsrc_t rk = rsrc(K, bytes), rv = rsrc(V, bytes);
-    const int k0 = i < n ? min((t0 + 2 * i) * BKV, a.Sk - BKV) : 0;
-    const uint32_t sk = (uint32_t)(k0 * a.k_ss * 2), sv = (uint32_t)(k0 * a.v_ss * 2);
+  FaRows kw(K, t0 * BKV, a.Sk, a.k_ss, D, 2 * BKV), vw(V, t0 * BKV, a.Sk, a.v_ss, D, 2 * BKV);
+  auto dma_tile = [&](lds_u16* st, int i) {  // (i: one after another)
+    const __amdgpu_buffer_rsrc_t rk = kw.next(i < n), rv = vw.next(i < n);
     lds_u16* sd = st + wave * 2 * TILE;
 #pragma unroll
     for (int q = 0; q < NDMA; ++q) {
-      dma16_lds(rk, kv_off[q], sk, (lds_void*)(sd + q * 512));
-      dma16_lds(rv, vv_off[q], sv, (lds_void*)(sd + (TILE + q * 512)));
+      dma16_lds(rk, kv_off[q], 0, (lds_void*)(sd + q * 512));
+      dma16_lds(rv, vv_off[q], 0, (lds_void*)(sd + (TILE + q * 512)));
     }
   };
 
@@ -1085,13 +1093,12 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
     const float mr = fa_round_max<ROUND>(sacc);
     const int k0 = (t0 + 2 * i) * BKV;
     float alpha;
-    const int kb0 = min(k0, a.Sk - BKV);
-    if (plain && k0 == kb0)
-      fa_softmax_tile<DT, FA_PLAIN>(a, kb0, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    if (plain && k0 + BKV <= a.Sk)
+      fa_softmax_tile<DT, FA_PLAIN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     else if (plain)
-      fa_softmax_tile<DT, FA_TAIL>(a, kb0, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+      fa_softmax_tile<DT, FA_TAIL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     else
-      fa_softmax_tile<DT, FA_GENERAL>(a, kb0, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+      fa_softmax_tile<DT, FA_GENERAL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     fa_rescale<DT>(o, alpha);
     l_run = __fadd_rn(l_run, fa_row_sum(pk));
 #pragma unroll
@@ -1185,8 +1192,8 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
   }
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
   typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-  const __amdgpu_buffer_rsrc_t ro = rsrc((uint64_t)(uintptr_t)g_dec_o, (uint32_t)(kDecWs * 4));
-  const __amdgpu_buffer_rsrc_t rm = rsrc((uint64_t)(uintptr_t)g_dec_ml, (uint32_t)(kDecWs / 4));
+  const __amdgpu_buffer_rsrc_t ro = fa_rsrc(g_dec_o, (uint32_t)(kDecWs * 4));
+  const __amdgpu_buffer_rsrc_t rm = fa_rsrc(g_dec_ml, (uint32_t)(kDecWs / 4));
   const uint32_t first = (uint32_t)(pair * splits);
   const uint32_t so = (uint32_t)(rows * D * 4), sm = (uint32_t)(rows * 8);  // bytes per split
   for (int x = tid * 4; x < rows * D; x += 512) {
@@ -1262,9 +1269,9 @@ static void launch_flash_d(const FlashArgs& a, bool buf, unsigned grid, hipStrea
 
 // Kernel choice for head dims 64 and 128 when every key tile is whole and
 // every K / V byte offset fits the buffer descriptors' 31 bits; other
-// shapes run the single-group kernel (ragged key counts through ping-pong,
-// the last tile moved back, measured 5 to 50 % slower below 1500 keys: half
-// the workgroups, and the mask's tile in the longer general form).  REW_MI355X_FLASH = single or pp
+// shapes run the single-group kernel (ragged key counts through ping-pong
+// measured 5 to 50 % slower below 1500 keys: half the workgroups, and the
+// mask's tile in the longer general form).  REW_MI355X_FLASH = single or pp
 // forces one (tests compare them).
 enum { FA_K_SINGLE = 0, FA_K_PP = 1, FA_K_DEC = 2 };
 static int flash_forced() {
@@ -1376,7 +1383,7 @@ void launch_flash(const FlashArgs& a, hipStream_t stream) {
     return;
   }
   const unsigned grid = (unsigned)(nqt * a.B * a.H);
-  const bool buf = a.Sk >= fa::BKV && flash_buf_ok(a);
+  const bool buf = flash_buf_ok(a);
   switch (a.D) {
     case 32: launch_flash_d<32>(a, buf, grid, stream); break;
     case 64: launch_flash_d<64>(a, buf, grid, stream); break;

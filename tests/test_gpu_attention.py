@@ -158,6 +158,37 @@ def test_flash_masked_keys_do_not_leak(gpu, oracle):
     assert not np.array_equal(a[:, :, :128], b[:, :, :128])
 
 
+@pytest.mark.parametrize("Sq,kernel", [(40, "flash_attn["), (1, "flash_attn_dec")])
+@pytest.mark.parametrize("Sk,D", [(129, 128), (300, 64), (191, 32), (1001, 128), (50, 64)])
+def test_flash_infinite_values_over_ragged_keys(gpu, oracle, Sq, kernel, Sk, D):
+    """An infinite V is an infinity in its output column, and the other columns
+    keep their bits: nothing that fills up a ragged last key tile (keys seen
+    before, what the LDS held) reaches the products with its zero
+    probabilities, where an infinity would make a NaN."""
+    B, H, Hkv = 2, 4, 2
+    q, k, v = _qkv(oracle, 31 + Sk, B, H, Hkv, Sq, Sk, D)
+    qt, kt = E.fromHost(q, DType.BFLOAT16), E.fromHost(k, DType.BFLOAT16)
+
+    def run(vals):
+        return _run(lambda: nn.scaledDotProductAttention(
+            qt, _expand(kt, B, Hkv, 2, Sk, D),
+            _expand(E.fromHost(vals, DType.BFLOAT16), B, Hkv, 2, Sk, D)))
+
+    first, last = max(0, Sk - 64), max(1, Sk // 64 * 64) - 1
+    want, names = run(v)
+    assert any(n.startswith(kernel) for n in names) or Sk < 128, names
+    w = v.copy()
+    w[:, :, first, 3] = np.inf
+    w[:, :, last, 7] = -np.inf
+    w[:, 1, first:last + 1, 9] = np.inf
+    w[:, :, :63, 12] = np.inf  # a tile that held the same LDS before
+    w[:, :, Sk - 1, 15] = np.inf
+    for c, x in ((3, np.inf), (7, -np.inf), (12, np.inf), (15, np.inf)):
+        want[..., c] = x
+    want[:, 2:, :, 9] = np.inf
+    np.testing.assert_array_equal(run(w)[0], want)
+
+
 def test_flash_gqa_equals_mha_with_repeated_kv(gpu, oracle):
     """GQA read through the head map equals MHA on explicitly repeated K/V."""
     B, H, Hkv, S, D = 1, 8, 2, 96, 64
