@@ -65,16 +65,26 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.0f;  // max growth (natural log) absorbed without rescaling
 }  // namespace fa
 
-// cmp(i, j) as selects on the (uniform) predicate, not a branch per element
-__device__ __forceinline__ bool fa_visible(int cmp, int i, int j) {
-  const bool lt = i < j, eq = i == j;
-  return cmp == vm::CMP_EQ   ? eq
-         : cmp == vm::CMP_NE ? !eq
-         : cmp == vm::CMP_LT ? lt
-         : cmp == vm::CMP_LE ? (lt || eq)
-         : cmp == vm::CMP_GT ? !(lt || eq)
-                             : !lt;
-}
+// The keys j for which cmp(i, j) holds, as one range, or all but that range
+// (NE): an element costs a comparison and a select.  (Selects on the predicate
+// itself came out as branches around each element, 2000 of them in a kernel.)
+struct FaRange {
+  int lo;
+  uint32_t n;
+  float in, out;  // the mask's summand inside the range and outside
+  __device__ __forceinline__ FaRange(const FlashArgs& a, int i) {
+    const int c = a.cmp;
+    lo = c == vm::CMP_LT ? i + 1 : (c == vm::CMP_GT || c == vm::CMP_GE) ? 0 : i;
+    const int hi = c == vm::CMP_GT                            ? i
+                   : (c == vm::CMP_LT || c == vm::CMP_LE) ? 0x7fffffff
+                                                              : i + 1;
+    n = (uint32_t)(hi - lo);
+    const bool ne = c == vm::CMP_NE;
+    in = !a.mask ? 0.0f : ne ? a.mask_false : a.mask_true;
+    out = !a.mask ? 0.0f : ne ? a.mask_true : a.mask_false;
+  }
+  __device__ __forceinline__ float at(int j) const { return (uint32_t)(j - lo) < n ? in : out; }
+};
 
 // Every (query, key) pair of queries [q0, q1] x keys [k0, k1] (inclusive)
 // satisfies cmp; only the ordered predicates can be decided from corners.
@@ -276,17 +286,15 @@ __device__ __forceinline__ void fa_softmax_tile(const FlashArgs& a, int k0, int 
       }
     mt = fa_max3(m0, m1, -INFINITY);
   } else {
+    const FaRange vis(a, qi);
     float m0 = -INFINITY;
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 16; e += 2) {
         const int j0 = k0 + kb * 32 + (e >> 2) * 8 + g * 4 + (e & 3);
-        float x0 = sacc_in[kb][e] * a.scale, x1 = sacc_in[kb][e + 1] * a.scale;
-        if (a.mask) {
-          x0 += fa_visible(a.cmp, qi, j0) ? a.mask_true : a.mask_false;
-          x1 += fa_visible(a.cmp, qi, j0 + 1) ? a.mask_true : a.mask_false;
-        }
+        float x0 = sacc_in[kb][e] * a.scale + vis.at(j0);
+        float x1 = sacc_in[kb][e + 1] * a.scale + vis.at(j0 + 1);
         x0 = j0 < a.Sk ? x0 * kLog2e : -INFINITY;
         x1 = j0 + 1 < a.Sk ? x1 * kLog2e : -INFINITY;
         t[kb][e] = x0;
@@ -1075,6 +1083,7 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
   float m_run = -INFINITY, l_run = 0.0f;
   const float sl2 = a.scale * kLog2e;
   const bool plain = !a.mask && a.scale > 0.0f;
+  const FaKinds kinds = fa_kinds(a, 0, a.Sq - 1);
 
   auto compute = [&](lds_u16* st, int i) __attribute__((always_inline)) {
     f32x16_t sacc[2];
@@ -1093,10 +1102,13 @@ __global__ void __launch_bounds__(128, 1) flash_dec_kernel(FlashArgs a, int spli
     const float mr = fa_round_max<ROUND>(sacc);
     const int k0 = (t0 + 2 * i) * BKV;
     float alpha;
-    if (plain && k0 + BKV <= a.Sk)
+    const int kind = fa_kind(kinds, t0 + 2 * i);
+    if (kind == FA_PLAIN)
       fa_softmax_tile<DT, FA_PLAIN>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     else if (plain)
       fa_softmax_tile<DT, FA_TAIL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
+    else if (kind == FA_DIAG_UP)
+      fa_softmax_tile<DT, FA_DIAG_UP>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     else
       fa_softmax_tile<DT, FA_GENERAL>(a, k0, qi, g, sl2, sacc, mr, pk, m_run, l_run, alpha);
     fa_rescale<DT>(o, alpha);
@@ -1296,9 +1308,15 @@ static bool flash_buf_ok(const FlashArgs& a) {
 // 103 us against 108); with two or more this one was ahead at every size
 // measured (64 x 32 / 8 heads x 300 keys 53 -> 28 us, 16 x 32 / 8 heads x 128
 // keys 10.9 -> 9.1).
+static bool hides_past_diagonal(const FlashArgs& a) { return a.skip && a.cmp == vm::CMP_GE; }
 static bool flash_dec_ok(const FlashArgs& a) {
   const int64_t pairs = (int64_t)a.B * a.Hkv;
   const bool fill = a.H > a.Hkv || (pairs <= 128 && a.Sk >= 8 * fa::BKV);
+  // Queries that see no key past their own leave one key tile: up to 512
+  // (batch, head) pairs the other kernels, which skip the rest too, finish it
+  // in one round and sooner (1 x 8 heads x 4096 keys 7.8 us against 8.9;
+  // 32 x 32 / 8 heads 14.8 against 12).
+  if (hides_past_diagonal(a) && (int64_t)a.B * a.H < 512) return false;
   return fill && (int64_t)(a.H / a.Hkv) * a.Sq <= fa::kDecCols && a.Sk >= 2 * fa::BKV &&
          pairs < (1 << 20) && a.k_ss >= 0 && a.v_ss >= 0 &&
          ((int64_t)a.Sk * a.k_ss + a.D) * 2 < (1ll << 31) &&
@@ -1347,10 +1365,13 @@ void launch_flash(const FlashArgs& a, hipStream_t stream) {
   const int kind = flash_kernel_kind(a);
   if (kind == FA_K_DEC) {
     int splits = 1, per = 1;
-    flash_dec_plan(a, &splits, &per);
+    // (at most 32 queries: where they see no key past their own, one tile is all)
+    FlashArgs d = a;
+    if (hides_past_diagonal(a)) d.Sk = std::min(a.Sk, fa::BKV);
+    flash_dec_plan(d, &splits, &per);
     const unsigned grid = (unsigned)(a.B * a.Hkv * splits);
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(grid), dim3(128), 0, stream, a, splits, per);
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(128), 0, stream, d, splits, per);
     };
     if (a.D == 32) {
       if (a.round_scores) go(flash_dec_kernel<32, true>);
