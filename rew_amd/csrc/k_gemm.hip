@@ -1335,12 +1335,13 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t 
   }
 }
 
-// f32 operands and result, and index arithmetic that fits 32 bits.
+// f32 operands and result, index arithmetic that fits 32 bits, and a launch
+// that HIP takes (fewer than 2^32 threads in x, 256 per tile).
 static bool f32_mfma_ok(const GemmArgs& g) {
   constexpr int64_t kLim = (int64_t)1 << 30;
   return g.dtype == REW_DT_FLOAT32 && g.c_dtype == REW_DT_FLOAT32 && g.K > 0 && g.M < kLim &&
          g.N < kLim && g.K < kLim &&
-         ((g.M + kFT - 1) / kFT) * ((g.N + kFT - 1) / kFT) * g.batch < kLim &&
+         ((g.M + kFT - 1) / kFT) * ((g.N + kFT - 1) / kFT) * g.batch < (1 << 24) &&
          g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE;
 }
 

@@ -79,3 +79,17 @@ def test_batches_and_epilogues(gpu):
         out, names = run(fn)
         assert len(names) == 1 and names[0].startswith("gemm_generic_mfma+bias"), names
         np.testing.assert_array_equal(out, ref)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (2, 4, 4)])
+def test_batch_past_the_grid_limit(gpu, M, K, N):
+    """2^24 products: more workgroups of 256 threads than one grid dimension takes."""
+    r = np.random.default_rng(K)
+    B = 1 << 24
+    a, b = (np.resize(r.standard_normal((4099, *s)).astype(np.float32), (B, *s))
+            for s in ((M, K), (K, N)))
+    got = E.toHost(O.dotGeneral(dev(a), dev(b), [0], [0], [2], [1]))
+    want = E.toHost(O.dotGeneral(dev(a[:4099]), dev(b[:4099]), [0], [0], [2], [1]))
+    for i in range(0, B, 4099):
+        part = got[i:i + 4099]
+        np.testing.assert_array_equal(part, want[:len(part)])
