@@ -1139,7 +1139,8 @@ constexpr int kFT = 64, kFK = 32;  // tile columns (rows: RW times), k-tile
 constexpr int kFG = 8;             // k-steps per group of LDS reads
 // From this many 128-row tiles (four per CU) the 32 x 32 blocks are faster:
 // 8192 x 2048 x 2048 658 us against 710, 1000 x 1000 x 3000 (376 tiles) 91
-// against 82.
+// against 82.  Not where a product has one row tile: 30000 products of 64 x 8 x
+// 64 271 us against 127.
 constexpr int64_t kF32TwoTiles = 1024;
 
 template <int RW, int AM, int BM>
@@ -1335,6 +1336,36 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t 
   }
 }
 
+// Which operands the kernel reads in 16-byte loads.
+struct F32Forms {
+  bool a_k, b_k, b_n;
+};
+static F32Forms f32_forms(const GemmArgs& g) {
+  auto vec = [&](const void* p, int64_t sb, int64_t s) {
+    return ((uintptr_t)p & 15) == 0 && sb % 4 == 0 && s % 4 == 0;
+  };
+  return {g.a_sk == 1 && g.K % 4 == 0 && vec(g.a, g.a_sb, g.a_sm),
+          g.b_sk == 1 && g.K % 4 == 0 && vec(g.b, g.b_sb, g.b_sn),
+          g.b_sn == 1 && g.N % 4 == 0 && vec(g.b, g.b_sb, g.b_sk)};
+}
+
+// Products of one tile that gemm_generic_kernel finishes sooner: it loads what
+// the product holds where this one's 4-byte loads fill the tile with repeats.
+// us for 60000 products (M x K x N), generic against this kernel: 1 x 1 x 1 215
+// / 518, 64 x 7 x 1 363 / 535, 1 x 7 x 64 289 / 365, 33 x 7 x 33 555 / 587, 2 x
+// 33 x 2 608 / 736, 3 x 8 x 3 308 / 373; past these lines 5 x 17 x 5 584 / 593
+// and 33 x 8 x 33 570 / 475, and with 16-byte loads on both sides 8 x 8 x 8 323
+// / 231.
+static bool f32_generic_better(const GemmArgs& g) {
+  if (g.M > kFT || g.N > kFT) return false;
+  const F32Forms f = f32_forms(g);
+  const int vecs = f.a_k + (f.b_k || f.b_n);
+  const int64_t mn = g.M * g.N;
+  if (vecs == 2) return false;
+  if (vecs == 1) return g.K < 8 || (g.K == 8 && mn <= 256);
+  return g.K <= 16 || (g.K <= 48 && mn <= 16);
+}
+
 // f32 operands and result, index arithmetic that fits 32 bits, and a launch
 // that HIP takes (fewer than 2^32 threads in x, 256 per tile).
 static bool f32_mfma_ok(const GemmArgs& g) {
@@ -1342,20 +1373,15 @@ static bool f32_mfma_ok(const GemmArgs& g) {
   return g.dtype == REW_DT_FLOAT32 && g.c_dtype == REW_DT_FLOAT32 && g.K > 0 && g.M < kLim &&
          g.N < kLim && g.K < kLim &&
          ((g.M + kFT - 1) / kFT) * ((g.N + kFT - 1) / kFT) * g.batch < (1 << 24) &&
-         g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE;
+         g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE && !f32_generic_better(g);
 }
 
 static void launch_gemm_f32_mfma(const GemmArgs& g, hipStream_t stream) {
-  auto vec = [&](const void* p, int64_t sb, int64_t s) {
-    return ((uintptr_t)p & 15) == 0 && sb % 4 == 0 && s % 4 == 0;
-  };
   int64_t tm = (g.M + 2 * kFT - 1) / (2 * kFT);
   const int64_t tn = (g.N + kFT - 1) / kFT;
-  const bool two = tm * tn * g.batch >= kF32TwoTiles;
+  const bool two = g.M > kFT && tm * tn * g.batch >= kF32TwoTiles;
   if (!two) tm = (g.M + kFT - 1) / kFT;
-  const bool avk = g.a_sk == 1 && g.K % 4 == 0 && vec(g.a, g.a_sb, g.a_sm);
-  const bool bvk = g.b_sk == 1 && g.K % 4 == 0 && vec(g.b, g.b_sb, g.b_sn);
-  const bool bvn = g.b_sn == 1 && g.N % 4 == 0 && vec(g.b, g.b_sb, g.b_sk);
+  const F32Forms f = f32_forms(g);
   const dim3 grid((unsigned)(tm * tn * g.batch));
 #define REW_F32_MFMA(AM, BM)                                                                     \
   do {                                                                                          \
@@ -1366,13 +1392,13 @@ static void launch_gemm_f32_mfma(const GemmArgs& g, hipStream_t stream) {
       hipLaunchKernelGGL((gemm_f32_mfma_kernel<1, AM, BM>), grid, dim3(256), 0, stream, g, tm,  \
                          tn);                                                                   \
   } while (0)
-  if (avk) {
-    if (bvn) REW_F32_MFMA(VEC_K, VEC_N);
-    else if (bvk) REW_F32_MFMA(VEC_K, VEC_K);
+  if (f.a_k) {
+    if (f.b_n) REW_F32_MFMA(VEC_K, VEC_N);
+    else if (f.b_k) REW_F32_MFMA(VEC_K, VEC_K);
     else REW_F32_MFMA(VEC_K, ANY);
   } else {
-    if (bvn) REW_F32_MFMA(ANY, VEC_N);
-    else if (bvk) REW_F32_MFMA(ANY, VEC_K);
+    if (f.b_n) REW_F32_MFMA(ANY, VEC_N);
+    else if (f.b_k) REW_F32_MFMA(ANY, VEC_K);
     else REW_F32_MFMA(ANY, ANY);
   }
 #undef REW_F32_MFMA

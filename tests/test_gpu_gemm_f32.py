@@ -93,3 +93,42 @@ def test_batch_past_the_grid_limit(gpu, M, K, N):
     for i in range(0, B, 4099):
         part = got[i:i + 4099]
         np.testing.assert_array_equal(part, want[:len(part)])
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (1, 1, 1, "gemm_generic"), (64, 7, 1, "gemm_generic"), (1, 7, 64, "gemm_generic"),
+    (3, 8, 3, "gemm_generic"), (2, 33, 2, "gemm_generic"), (13, 16, 13, "gemm_generic_mfma"),
+    (13, 15, 13, "gemm_generic"), (13, 17, 13, "gemm_generic_mfma"),
+    (8, 8, 8, "gemm_generic_mfma"), (65, 7, 3, "gemm_generic_mfma"),
+    (64, 8, 64, "gemm_generic_mfma"),
+])
+def test_batches_of_small_products(gpu, M, K, N, kernel):
+    """Which kernel takes 1500 products of one tile each, and its sums."""
+    r = np.random.default_rng(M + K + N)
+    a, b = (r.standard_normal((1500, *s)).astype(np.float32) for s in ((M, K), (K, N)))
+    got, names = run(lambda: O.dotGeneral(dev(a), dev(b), [0], [0], [2], [1]))
+    assert [n.split("[")[0] for n in names] == [kernel], names
+    want = np.matmul(a.astype(np.float64), b.astype(np.float64))
+    bound = (K + 1) * 2.0 ** -24 * np.matmul(np.abs(a).astype(np.float64), np.abs(b))
+    assert np.all(np.abs(got - want) <= bound)
+
+
+def test_one_row_tile_keeps_its_height(gpu):
+    """Many products of at most 64 rows run 64-row tiles: about twice the rate of
+    128-row ones, which hold twice the LDS and load as much again for nothing."""
+    def us(M):
+        a, b = E.empty(E.DType.FLOAT32, (30000, M, 8)), E.empty(E.DType.FLOAT32, (30000, 8, 32))
+        best = 1e9
+        for _ in range(5):
+            E.profileBegin()
+            out = O.dotGeneral(a, b, [0], [0], [2], [1])
+            E.flush()
+            prof = E.profileEnd()
+            del out
+            assert len(prof) == 1 and prof[0][0].startswith("gemm_generic_mfma"), prof
+            best = min(best, prof[0][2] * 1e3)
+        return best
+
+    # (measured: 127 us against 313; in 128-row tiles 288)
+    low, high = us(32), us(100)
+    assert low <= 0.65 * high, (low, high)
