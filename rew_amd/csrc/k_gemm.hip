@@ -1407,14 +1407,29 @@ static void launch_gemm_f32_mfma(const GemmArgs& g, hipStream_t stream) {
 // Problems whose 64x64 tiles would leave most CUs idle run 16x16 tiles, until
 // those fill the CUs several times over.  The matrix-core kernel takes about
 // 6 us + 24 ns per k-step whatever its tiles leave idle; the 16x16 tiles are
-// ahead of that up to 32 tiles of 64x64 (128 x 1024 x 1024: 29 us against 31;
-// 333 x 1024 x 512: 46 against 31), or 80 where K is short (333 x 256 x 512:
-// 12 against 14), and no more once K passes the slab they hold in LDS
-// (333 x 2816 x 1024: 178 against 71).
+// ahead of that
+//   * up to 32 tiles of 64x64 (128 x 1024 x 1024: 29 us against 31; 333 x 1024
+//     x 512: 46 against 31), or 80 where K is short (333 x 256 x 512: 12 against
+//     14);
+//   * for few rows, which leave the 64x64 tiles mostly empty, while the CUs hold
+//     the slabs of all of them at once (8 x 1024 x 2816: 15 against 28, 32 x 512
+//     x 4096 12 / 17, 16 x 1024 x 4096 17 / 28; with more 17 x 1024 x 4096 35 /
+//     28, 64 x 512 x 2816 19 / 17);
+//   * where K passes the slab, with a tile per CU, for at most 8 rows (1 x 4096 x
+//     4096: 87 against 95, 8 x 2048 x 1024 48 / 51, 16 x 2048 x 1024 52 / 51)
+//     or operands that the matrix-core kernel reads 4 bytes at a time (100 x
+//     10000 x 70: 239 / 345); otherwise no more (333 x 2816 x 1024: 178 / 71).
 static bool small_ok(const GemmArgs& g) {
   const int64_t tiles64 = ((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
-  if (f32_mfma_ok(g)) return g.K <= kSmallWholeK && tiles64 <= (g.K >= 512 ? 32 : 80);
-  return tiles64 < 128 && g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE;
+  if (!f32_mfma_ok(g)) return tiles64 < 128 && g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE;
+  const int64_t tiles16 = ((g.M + 15) / 16) * ((g.N + 15) / 16) * g.batch;
+  if (g.K > kSmallWholeK) {
+    const F32Forms f = f32_forms(g);
+    return tiles16 <= 256 && (g.M <= 8 || !f.a_k || !(f.b_k || f.b_n));
+  }
+  const int64_t slabs = 16 * (((g.K + 15) & ~(int64_t)15) + 4) * 4 * 2;
+  return tiles64 <= (g.K >= 512 ? 32 : 80) ||
+         (g.K >= 512 && tiles16 <= 256 * (160 * 1024 / slabs));
 }
 
 static bool mfma_ok(const GemmArgs& g, bool* a_kc, bool* b_kc) {

@@ -132,3 +132,21 @@ def test_one_row_tile_keeps_its_height(gpu):
     # (measured: 127 us against 313; in 128-row tiles 288)
     low, high = us(32), us(100)
     assert low <= 0.65 * high, (low, high)
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (8, 1024, 2816, "gemm_f32_small"), (16, 1024, 4096, "gemm_f32_small"),
+    (17, 1024, 4096, "gemm_generic_mfma"), (32, 512, 4096, "gemm_f32_small"),
+    (33, 512, 4096, "gemm_generic_mfma"), (1, 4096, 4096, "gemm_f32_small"),
+    (8, 2048, 1024, "gemm_f32_small"), (9, 2048, 1024, "gemm_generic_mfma"),
+    (100, 3000, 70, "gemm_f32_small"), (100, 3000, 72, "gemm_generic_mfma"),
+])
+def test_few_rows(gpu, M, K, N, kernel):
+    """Which kernel takes a product of few rows, and its sums."""
+    r = np.random.default_rng(M + K + N)
+    a, b = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    got, names = run(lambda: O.matmul(dev(a), dev(b)))
+    assert [n.split("[")[0] for n in names] == [kernel], names
+    want = a.astype(np.float64) @ b
+    bound = (K + 1) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b))
+    assert np.all(np.abs(got - want) <= bound)
