@@ -1153,7 +1153,7 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t 
   __shared__ __attribute__((aligned(16))) float As[2][FM][KP];
   __shared__ __attribute__((aligned(16))) float Bs[2][BK_ROWS ? kFT * KP : kFK * NP];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  const int M = (int)g.M, N = (int)g.N, K = (int)g.K, K16 = (K + 15) & ~15;
 
   // XCD-contiguous ranges, then groups of 8 row tiles walked down the columns
   int64_t t = blockIdx.x, b;
@@ -1218,6 +1218,19 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t 
     const float* ra = rga[set];
     const float* rb = rgb[set];
     auto keep = [&](float v, int k) { return vm::as_f(vm::as_u(v) & (uint32_t)((k - K) >> 31)); };
+    // B's zeros are negative from the next multiple of 16 on, where the other
+    // kernels' chains end: 0 * -0 leaves a sum of -0 (of products that underflow)
+    // as it is, where 0 * 0 would make it +0.  (One bit-field insert in place of
+    // keep's and; z from the slot's k in the tile, which the loop does not change.)
+    const uint32_t neg = K16 & 16 ? 0x80000000u : 0u;
+    auto keep_b = [&](float v, int k, int kin) {
+      const uint32_t m = (uint32_t)((k - K) >> 31), z = kin >= 16 ? neg : 0u;
+      return vm::as_f((vm::as_u(v) & m) | (z & ~m));
+    };
+    auto keep4_b = [&](const float* v, int k, int kin) {
+      return make_float4(keep_b(v[0], k, kin), keep_b(v[1], k, kin), keep_b(v[2], k, kin),
+                         keep_b(v[3], k, kin));
+    };
     auto keep4 = [&](const float* v, int k) {
       return make_float4(keep(v[0], k), keep(v[1], k), keep(v[2], k), keep(v[3], k));
     };
@@ -1235,12 +1248,13 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t 
     for (int i = 0; i < (BM == ANY ? 8 : 2); ++i) {
       const int e = tid + i * 256;
       if constexpr (BM == VEC_K) {
-        *(float4*)&Bs[s][(e >> 3) * KP + (e & 7) * 4] = keep4(rb + 4 * i, k0 + (e & 7) * 4);
+        *(float4*)&Bs[s][(e >> 3) * KP + (e & 7) * 4] = keep4_b(rb + 4 * i, k0 + (e & 7) * 4, (e & 7) * 4);
       } else if constexpr (BM == VEC_N) {
-        *(float4*)&Bs[s][(e >> 4) * NP + (e & 15) * 4] = keep4(rb + 4 * i, k0 + (e >> 4));
+        *(float4*)&Bs[s][(e >> 4) * NP + (e & 15) * 4] =
+            keep4_b(rb + 4 * i, k0 + (e >> 4), 16 * i);
       } else {
         const int k = b_k ? e & 31 : e >> 6;
-        Bs[s][k * NP + (b_k ? e >> 5 : e & 63)] = keep(rb[i], k0 + k);
+        Bs[s][k * NP + (b_k ? e >> 5 : e & 63)] = keep_b(rb[i], k0 + k, k);
       }
     }
   };

@@ -150,3 +150,21 @@ def test_few_rows(gpu, M, K, N, kernel):
     want = a.astype(np.float64) @ b
     bound = (K + 1) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b))
     assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("K", [16, 48, 40, 32, 12])
+def test_products_that_underflow(gpu, form, K):
+    """Sums of denormals, and zeros whose sign is the last term's: a chain ends
+    at the next multiple of 16 in every kernel, with zero terms past K."""
+    _, f = FORMS[form]
+    a = np.full((640, K), -1e-20, np.float32)
+    b = np.full((K, 648), 1e-20, np.float32)
+    b[:, ::2] = 1e-30  # (the products underflow)
+    got, names = run(lambda: f(a, b))
+    assert any(n.startswith("gemm_generic_mfma") for n in names), names
+    ref, names = run(lambda: f(a[:33], b[:, :65]))
+    assert any(n.startswith("gemm_f32_small") for n in names), names
+    np.testing.assert_array_equal(got[:33, :65].view(np.uint32), ref.view(np.uint32))
+    assert (ref[0, 0] == 0) and np.signbit(ref[0, 0]) == (K % 16 == 0)
+    assert 0 < -ref[0, 1] < 1e-37
