@@ -1279,6 +1279,7 @@ void Lower::emit_reduce(Node* n) {
       }
       x->plan_mat = true;
       ensure_mat(x);
+      if (out->st) return;  // (that found this reduction to store x in)
     }
   }
   throw Error(REW_MI355X_ERR_UNSUPPORTED, "reduction prologue too large");

@@ -700,3 +700,64 @@ def test_reduction_stores_the_chain_it_reads(gpu, compiled):
                         json.dumps(cases)], env=dict(os.environ, REW_MI355X_JIT=compiled),
                        capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, (r.stdout[-500:], r.stderr[-3000:])
+
+
+@pytest.mark.parametrize("held", [False, True])
+def test_reduction_of_a_chain_past_one_program(gpu, held):
+    """A chain of more leaves than a program takes is cut once, and its
+    reduction is one launch whether or not the chain is read on its own."""
+    r = np.random.default_rng(8)
+    xs = [r.integers(-8, 8, (1100, 256)).astype(np.float32) for _ in range(16)]
+
+    def fn():
+        y = E.fromHost(xs[0])
+        for x in xs[1:]:
+            y = O.add(y, E.fromHost(x))
+        outs = [O.reduceSum(y, [1])] + ([y] if held else [])
+        del y
+        E.flush()
+        return outs
+
+    E.profileBegin()
+    outs = fn()
+    names = [n for n, k, _ in E.profileEnd() for _ in range(k)]
+    assert sum(n.startswith("reduce") for n in names) == 1, names
+    want = np.sum(xs, 0)
+    np.testing.assert_array_equal(E.toHost(outs[0]), want.sum(1))
+    if held:
+        np.testing.assert_array_equal(E.toHost(outs[1]), want)
+
+
+@pytest.mark.parametrize("leaf", ["transposed", "rows", "reversed"])
+def test_kept_chain_of_a_view(gpu, leaf):
+    """The chain that a reduction stores may read transposed, cut or reversed
+    views: the same bits as op by op."""
+    r = np.random.default_rng(9)
+    x = r.standard_normal((1100, 256)).astype(np.float32)
+    src = np.ascontiguousarray(x.T) if leaf == "transposed" else r.standard_normal(
+        (1200, 300)).astype(np.float32) if leaf == "rows" else x
+    b = r.standard_normal((1100, 256)).astype(np.float32)
+
+    def fn():
+        t = E.fromHost(src)
+        if leaf == "transposed":
+            t = O.transpose(t, [1, 0])
+        elif leaf == "rows":
+            t = O.slice_(t, [7, 11], [1107, 267])
+        else:
+            t = E.dispatchEager("reverse", [t], [("dimensions", "[0, 1]")])[0]
+        y = nn.relu(O.add(t, E.fromHost(b)))
+        outs = [y, O.reduceSum(y, [1]), O.reduceMax(y, [1])]
+        E.flush()
+        return outs
+
+    E.profileBegin()
+    got = fn()
+    names = [n for n, _, _ in E.profileEnd()]
+    got = [E.toHost(t) for t in got]
+    E.setMode(E.MODE_OP_BY_OP)
+    want = [E.toHost(t) for t in fn()]
+    E.setMode(E.MODE_DEFERRED)
+    assert any(",kept" in n for n in names), names
+    for g, w in zip(got, want):
+        np.testing.assert_array_equal(g, w)
