@@ -442,7 +442,8 @@ struct StripPlan {
 int64_t col_tiles(const GemmArgs& g) { return (g.N + BN - 1) / BN; }
 
 // Row blocks per tile and splits of k, by an estimate of the time in
-// microseconds.  Its terms are fits to measurements over 8 .. 2000 rows of
+// microseconds (good enough to tell plans of one product apart; strip_time is
+// the one to compare with another kernel).  Its terms are fits to measurements over 8 .. 2000 rows of
 // K x N = 4096 x 4096, 14336 x 4096 and 4096 x 14336 (weights out of cache),
 // which they meet within about 15 %:
 //   * a k-tile of one workgroup per CU (more workgroups share the CU);
@@ -491,6 +492,33 @@ StripPlan plan_for(const GemmArgs* segs, int n) {
   return best;
 }
 
+// Time of a plan, and of the 256 x 256 kernel for the same product, in
+// microseconds: fits to both kernels' times over 8 .. 8000 rows, K 64 .. 14336
+// and N 512 .. 128256, which they meet within 8 % (half of them) to 20 % (nine
+// in ten).  A CU runs its workgroups' k-tiles one after another (two of them at
+// once up to 64 rows) and pays a workgroup's start and end once per round; the
+// 256 x 256 kernel likewise, a k-tile costing more with more CUs busy.
+double strip_time(const StripPlan& p, int64_t K, double weights, bool dual) {
+  constexpr double kTile[2][4] = {{0.230, 0.330, 0.510, 0.579}, {0.495, 0.579, 0.912, 1.094}};
+  constexpr double kEnds[2][4] = {{4.1, 4.8, 6.8, 7.7}, {5.3, 7.3, 10.3, 11.3}};
+  constexpr double kSum[2][4] = {{3.2, 4.0, 4.4, 6.1}, {4.2, 6.4, 7.9, 8.7}};
+  const int x = p.R == 1 ? 0 : p.R == 2 ? 1 : p.R == 4 ? 2 : 3;
+  const int64_t wgs = p.tiles_m * p.tiles_n * p.splits, slots = !dual && p.R <= 2 ? 512 : 256;
+  const double loop = (double)((wgs + 255) / 256) * p.per * kTile[dual][x] +
+                      (double)((wgs + slots - 1) / slots) * kEnds[dual][x];
+  const double hbm = dual ? 6.5e6 : 5.5e6, wg = dual ? 58e3 : 102e3, l2 = dual ? 14e6 : 15.6e6;
+  const double mem = weights / hbm + weights / (wg * (double)(wgs < slots ? wgs : slots)) +
+                     (double)(p.tiles_m - 1) * weights / l2;
+  return 3.8 + (loop > mem ? loop : mem) + (p.splits > 1 ? kSum[dual][x] : 0.0);
+}
+double tile256_time(int64_t tiles, int64_t K, double weights, bool dual) {
+  const double busy = tiles <= 96 ? 0.0 : tiles >= 256 ? 1.0 : (double)(tiles - 96) / 160;
+  const double step = dual ? 0.485 + 0.117 * busy : 0.48 + 0.04 * busy;  // 32 of K
+  const double loop =
+      (double)((tiles + 255) / 256) * ((dual ? 7.4 : 8.7) + (double)((K + 31) / 32) * step);
+  return (dual ? 7.1 : 6.4) + (loop > weights / 4.8e6 ? loop : weights / 4.8e6);
+}
+
 template <int R, bool DUAL, int NS, int OCC>
 void go(const GemmSegs& gs, const StripPlan& p, hipStream_t stream) {
   StripArgs sa{(int)p.tiles_m, (int)p.tiles_n, p.splits, p.per};
@@ -521,19 +549,21 @@ bool gemm_strip_better(const GemmArgs* segs, int n) {
   }
   tiles *= (f.M + 255) / 256;
   if (tiles >= 4096) return false;
-  // Fewer than 96 of the 256 x 256 kernel's tiles otherwise go to the
-  // 128 x 128 kernel, which no size measured had faster (8 x 14336 x 4096:
-  // 443 us against 28 here).  The 256 x 256 kernel takes a round in 0.55 us
-  // per 32 of K on half of the CUs and 0.72 on most of them, whatever the
-  // tiles hold, or the weights' time (2000 x 14336 x 4096: 247 us against 286
-  // here; 16 x 4096 x 128256: 227 us against 192).
-  if (tiles < 96 && n == 1 && !dual) return true;
+  // Fewer than 96 of the 256 x 256 kernel's tiles otherwise go to the 128 x 128
+  // kernel or, as SwiGLU, to the older 256 x 256 one, which no size measured had
+  // faster (8 x 14336 x 4096: 443 us against 28 here; SwiGLU 1500 x 2048 x 1408:
+  // 92 against 49).
+  if (tiles < 96 && n == 1) return true;
+  // From there on the two estimates decide, where they differ by more than
+  // their bias: the 256 x 256 kernel had every product of more than 256 rows
+  // (us here / there: 1000 x 1024 x 8192 31 / 29, 600 x 4096 x 14336 121 / 83,
+  // 3000 x 64 x 4096 26 / 17; SwiGLU 600 x 4096 x 14336 180 / 158, 300 x 4096 x
+  // 14336 98 / 92), this one the few rows over many weights (16 x 4096 x 128256
+  // 190 / 201, 8 x 1024 x 128256 52 / 66; SwiGLU 64 x 4096 x 14336 72 / 93).
   double weights = 0;
   for (int i = 0; i < n; ++i) weights += (dual ? 4.0 : 2.0) * (double)f.K * (double)segs[i].N;
-  const double loop = (double)((tiles + 255) / 256) * (double)((f.K + 31) / 32) *
-                      (tiles <= 160 ? 0.55 : 0.72);
-  const double big = 6 + (loop > weights / 4.6e6 ? loop : weights / 4.6e6);
-  return plan_for(segs, n).us < big;
+  const double here = strip_time(plan_for(segs, n), f.K, weights, dual);
+  return here < (dual && f.M > 64 ? 0.85 : 0.97) * tile256_time(tiles, f.K, weights, dual);
 }
 
 void launch_gemm_strip(const GemmArgs* segs, int n, hipStream_t stream) {

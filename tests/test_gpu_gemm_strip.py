@@ -117,3 +117,35 @@ def test_reversed_rows(gpu):
         got = E.toHostF32(O.matmul(flip(_dev(x)), _dev(w)))
         want = E.toHostF32(O.matmul(_dev(np.ascontiguousarray(x[::-1])), _dev(w)))
         assert np.linalg.norm(got - want) <= 2e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("M,K,N,strip", [
+    (1000, 1024, 8192, False), (600, 4096, 14336, False), (3000, 64, 4096, False),
+    (4000, 256, 1408, False), (1500, 4096, 4096, False), (1400, 4096, 4096, False),
+    (1200, 4096, 4096, True), (8, 1024, 128256, True), (16, 4096, 14336, True),
+])
+def test_strip_or_256_tiles(gpu, M, K, N, strip):
+    """Which kernel takes a Linear: the strip kernel below 96 tiles of 256x256,
+    and past that for few rows over many weights only."""
+    w, b = E.empty(DType.BFLOAT16, (K, N)), E.empty(DType.BFLOAT16, (N,))
+    E.profileBegin()
+    out = nn.Linear(w, b).forward(E.empty(DType.BFLOAT16, (M, K)))
+    E.flush()
+    names = [n for n, _, _ in E.profileEnd()]
+    del out
+    assert len(names) == 1 and ("_strip" in names[0]) == strip, names
+
+
+@pytest.mark.parametrize("T,H,I,strip", [
+    (300, 4096, 14336, False), (600, 4096, 14336, False), (6000, 2048, 1408, False),
+    (2600, 512, 2048, False), (64, 4096, 14336, True), (1500, 2048, 1408, True),
+])
+def test_swiglu_strip_or_256_tiles(gpu, T, H, I, strip):
+    e = lambda *s: E.empty(DType.BFLOAT16, s)  # noqa: E731
+    gate, up, down = (nn.Linear(e(*s), e(s[1])) for s in ((H, I), (H, I), (I, H)))
+    E.profileBegin()
+    out = nn.GatedFeedForward(gate, up, down).forward(e(1, T, H))
+    E.flush()
+    names = [n for n, _, _ in E.profileEnd()]
+    del out
+    assert [("_strip" in n) for n in names if "swiglu" in n] == [strip], names
