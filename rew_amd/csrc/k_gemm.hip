@@ -1529,7 +1529,7 @@ bool gemm_epilogue_ok(const GemmArgs& g) {
 
 const char* gemm_variant(const GemmArgs& g) {
   bool akc, bkc;
-  if (gemm_strip_better(&g, 1))
+  if (gemm_strip_plan(&g, 1).R)
     return g.epi == EPI_SWIGLU ? "gemm_lds_swiglu_strip" : "gemm_lds_nn_strip";
   if (use_lds(g)) {
     gemm_lds_ok(g, &bkc);
@@ -1546,11 +1546,11 @@ const char* gemm_variant(const GemmArgs& g) {
   return "gemm_bf16_mfma_nt";
 }
 
-void launch_gemm(const GemmArgs& g, hipStream_t stream) {
+void launch_gemm(const GemmArgs& g, const StripPlan& strip, hipStream_t stream) {
   if (g.M == 0 || g.N == 0 || g.batch == 0) return;
   bool akc, bkc;
-  if (gemm_strip_better(&g, 1)) {
-    launch_gemm_strip(&g, 1, stream);
+  if (strip.R) {
+    launch_gemm_strip(&g, 1, strip, stream);
     return;
   }
   if (use_lds(g)) {

@@ -1067,10 +1067,10 @@ bool gemm_multi_ok(const GemmArgs* segs, int n) {
   return true;
 }
 
-void launch_gemm_multi(const GemmArgs* segs, int n, hipStream_t stream) {
+void launch_gemm_multi(const GemmArgs* segs, int n, const StripPlan& strip, hipStream_t stream) {
   if (!gemm_multi_ok(segs, n)) fail(REW_MI355X_ERR_INVALID, "internal: GEMM set not launchable");
-  if (gemm_strip_better(segs, n)) {
-    launch_gemm_strip(segs, n, stream);
+  if (strip.R) {
+    launch_gemm_strip(segs, n, strip, stream);
     return;
   }
   GemmSegs gs;

@@ -433,12 +433,6 @@ __global__ void __launch_bounds__(256, OCC) gemm_strip_kernel(GemmSegs gs, Strip
 
 namespace {
 
-struct StripPlan {
-  int R, splits, per;
-  int64_t tiles_m, tiles_n;
-  double us;  // estimated time
-};
-
 int64_t col_tiles(const GemmArgs& g) { return (g.N + BN - 1) / BN; }
 
 // Row blocks per tile and splits of k, by an estimate of the time in
@@ -458,9 +452,8 @@ StripPlan plan_for(const GemmArgs* segs, int n) {
   const int64_t M = segs[0].M, K = segs[0].K;
   const bool dual = segs[0].epi == EPI_SWIGLU;
   const int64_t nk = (K + BK - 1) / BK;
-  StripPlan best{};
-  best.us = 1e30;
-  best.tiles_n = 0;
+  StripPlan best;
+  double best_us = 1e30;
   double weights = 0;
   for (int i = 0; i < n; ++i) {
     best.tiles_n += col_tiles(segs[i]);
@@ -480,8 +473,8 @@ StripPlan plan_for(const GemmArgs* segs, int n) {
       const double mem = weights / 8e6 + weights / (57e3 * (double)(wgs < 256 ? wgs : 256)) +
                          (double)(tm - 1) * weights / 13e6;
       const double us = 4 + (loop > mem ? loop : mem) + (s > 1 ? kSum[dual][x] : 0.0);
-      if (us < best.us) {
-        best.us = us;
+      if (us < best_us) {
+        best_us = us;
         best.R = kR[x];
         best.per = (int)per;
         best.splits = (int)((nk + per - 1) / per);
@@ -529,31 +522,33 @@ void go(const GemmSegs& gs, const StripPlan& p, hipStream_t stream) {
 
 }  // namespace
 
-bool gemm_strip_better(const GemmArgs* segs, int n) {
+StripPlan gemm_strip_plan(const GemmArgs* segs, int n) {
+  const StripPlan none;
   static const bool forced = std::getenv("REW_MI355X_GEMM_TILE") != nullptr;
-  if (forced || n < 1 || n > kMaxSegs) return false;
+  if (forced || n < 1 || n > kMaxSegs) return none;
   const GemmArgs& f = segs[0];
-  if (f.batch != 1 || f.M <= 0) return false;
+  if (f.batch != 1 || f.M <= 0) return none;
   const bool dual = f.epi == EPI_SWIGLU;
   constexpr int64_t kLim = (int64_t)1 << 31;
   int64_t tiles = 0;  // of the 256 x 256 kernel
   for (int i = 0; i < n; ++i) {
     const GemmArgs& g = segs[i];
     bool bkc;
-    if (!gemm_lds_ok(g, &bkc) || bkc || (g.epi == EPI_SWIGLU) != dual) return false;
-    if (g.epi == EPI_BIAS_RELU) return false;
+    if (!gemm_lds_ok(g, &bkc) || bkc || (g.epi == EPI_SWIGLU) != dual) return none;
+    if (g.epi == EPI_BIAS_RELU) return none;
     // 32-bit byte offsets from each operand's base
     if (((g.M - 1) * g.a_sm + g.K) * 2 >= kLim || ((g.K - 1) * g.b_sk + g.N) * 2 >= kLim)
-      return false;
+      return none;
     tiles += (g.N + (dual ? 127 : 255)) / (dual ? 128 : 256);
   }
   tiles *= (f.M + 255) / 256;
-  if (tiles >= 4096) return false;
+  if (tiles >= 4096) return none;
   // Fewer than 96 of the 256 x 256 kernel's tiles otherwise go to the 128 x 128
   // kernel or, as SwiGLU, to the older 256 x 256 one, which no size measured had
   // faster (8 x 14336 x 4096: 443 us against 28 here; SwiGLU 1500 x 2048 x 1408:
   // 92 against 49).
-  if (tiles < 96 && n == 1) return true;
+  const StripPlan p = plan_for(segs, n);
+  if (tiles < 96 && n == 1) return p;
   // From there on the two estimates decide, where they differ by more than
   // their bias: the 256 x 256 kernel had every product of more than 256 rows
   // (us here / there: 1000 x 1024 x 8192 31 / 29, 600 x 4096 x 14336 121 / 83,
@@ -562,15 +557,15 @@ bool gemm_strip_better(const GemmArgs* segs, int n) {
   // 190 / 201, 8 x 1024 x 128256 52 / 66; SwiGLU 64 x 4096 x 14336 72 / 93).
   double weights = 0;
   for (int i = 0; i < n; ++i) weights += (dual ? 4.0 : 2.0) * (double)f.K * (double)segs[i].N;
-  const double here = strip_time(plan_for(segs, n), f.K, weights, dual);
-  return here < (dual && f.M > 64 ? 0.85 : 0.97) * tile256_time(tiles, f.K, weights, dual);
+  const double here = strip_time(p, f.K, weights, dual);
+  const double there = tile256_time(tiles, f.K, weights, dual);
+  return here < (dual && f.M > 64 ? 0.85 : 0.97) * there ? p : none;
 }
 
-void launch_gemm_strip(const GemmArgs* segs, int n, hipStream_t stream) {
+void launch_gemm_strip(const GemmArgs* segs, int n, const StripPlan& p, hipStream_t stream) {
   GemmSegs gs;
   std::memset(&gs, 0, sizeof gs);
   gs.n = n;
-  const StripPlan p = plan_for(segs, n);
   for (int i = 0; i < n; ++i) {
     gs.g[i] = segs[i];
     gs.tn0[i + 1] = gs.tn0[i] + col_tiles(segs[i]);

@@ -110,7 +110,21 @@ enum GemmEpi : int {
   EPI_NONE = 0, EPI_BIAS = 1, EPI_BIAS_RES = 2, EPI_SWIGLU = 3, EPI_BIAS_ROPE = 4,
   EPI_BIAS_RELU = 5
 };
-void launch_gemm(const GemmArgs& g, hipStream_t stream);
+
+// How the strip kernel (k_gemm_strip.hip: bf16 products of few rows or few
+// tiles) takes a product or set: 32 R rows per tile, k split over `splits`
+// workgroups of `per` k-tiles each.  R = 0: another kernel takes it.
+struct StripPlan {
+  int R = 0, splits = 1, per = 0;
+  int64_t tiles_m = 0, tiles_n = 0;
+};
+// The plan depends on shapes, strides and alignments alone, so a recorded
+// launch keeps it.
+StripPlan gemm_strip_plan(const GemmArgs* segs, int n);
+void launch_gemm_strip(const GemmArgs* segs, int n, const StripPlan& plan, hipStream_t stream);
+
+// strip: gemm_strip_plan's answer for g.
+void launch_gemm(const GemmArgs& g, const StripPlan& strip, hipStream_t stream);
 
 // Grouped GEMM over packed rows (the routed experts of a MoE layer).  Group
 // i owns packed rows [off[i], off[i+1]) and row tiles
@@ -172,12 +186,7 @@ struct GemmSegs {
   GemmArgs g[kMaxSegs];
 };
 bool gemm_multi_ok(const GemmArgs* segs, int n);
-void launch_gemm_multi(const GemmArgs* segs, int n, hipStream_t stream);
-// The strip kernel (k_gemm_strip.hip) for bf16 products of few rows or few
-// tiles; `better` also says whether it takes the set (same conditions as
-// gemm_multi_ok, N-contiguous B) in place of the 256x256 kernels.
-bool gemm_strip_better(const GemmArgs* segs, int n);
-void launch_gemm_strip(const GemmArgs* segs, int n, hipStream_t stream);
+void launch_gemm_multi(const GemmArgs* segs, int n, const StripPlan& strip, hipStream_t stream);
 // Whether launch_gemm runs g with its epilogue (EPI_SWIGLU needs the large
 // dual kernel; the others run on every MFMA kernel).
 bool gemm_epilogue_ok(const GemmArgs& g);

@@ -179,8 +179,12 @@ struct Exec {
   void operator()(EwL& l) { launch_ew(l.P, l.S, l.vec, c->stream); }
   void operator()(ReduceL& l) { launch_reduce(l.P, l.S, l.A, l.vec, c->stream); }
   void operator()(GemmL& l) {
-    if (l.multi) launch_gemm_multi(l.g.data(), (int)l.g.size(), c->stream);
-    else launch_gemm(l.g[0], c->stream);
+    if (!l.planned) {
+      l.strip = gemm_strip_plan(l.g.data(), (int)l.g.size());
+      l.planned = true;
+    }
+    if (l.multi) launch_gemm_multi(l.g.data(), (int)l.g.size(), l.strip, c->stream);
+    else launch_gemm(l.g[0], l.strip, c->stream);
   }
   void operator()(FlashArgs& a) { launch_flash(a, c->stream); }
   void operator()(RowNormArgs& a) { launch_rmsnorm_rows(a, c->stream); }

@@ -32,6 +32,8 @@ struct ReduceL {
 struct GemmL {
   std::vector<GemmArgs> g;  // one GEMM, or the segments of a multi-segment launch
   bool multi;
+  StripPlan strip;  // chosen once, at the first launch
+  bool planned = false;
 };
 struct IndexMapL {
   IndexMapArgs g;
