@@ -1106,9 +1106,23 @@ __global__ void __launch_bounds__(256) gemm_f32_narrow_kernel(GemmArgs g) {
   }
 }
 
+// REW_MI355X_GEMM_TILE forces a kernel where it can run: "256", "128" or "lds"
+// (the direct-to-LDS kernels) for bf16 products, so that tests reach the large
+// tiles' tails at small sizes, "generic" for f32 ones, so that they have the
+// other kernels' reference.  Unset picks by size.
+static int forced_tile() {
+  static const int v = [] {
+    const char* s = std::getenv("REW_MI355X_GEMM_TILE");
+    if (s && std::string(s) == "lds") return 1;
+    if (s && std::string(s) == "generic") return 2;
+    return s ? std::atoi(s) : 0;
+  }();
+  return v;
+}
+
 static bool f32_narrow_ok(const GemmArgs& g) {
-  return g.dtype == REW_DT_FLOAT32 && g.batch == 1 && g.M >= 1 && g.N >= 4 && g.N <= 64 &&
-         g.N % 4 == 0 && g.K >= 64 && g.K % 64 == 0 && g.a_sk == 1 && g.b_sn == 1 &&
+  return forced_tile() != 2 && g.dtype == REW_DT_FLOAT32 && g.batch == 1 && g.M >= 1 &&
+         g.N >= 4 && g.N <= 64 && g.N % 4 == 0 && g.K >= 64 && g.K % 64 == 0 && g.a_sk == 1 && g.b_sn == 1 &&
          g.a_sm % 4 == 0 && g.b_sk % 4 == 0 && ((uintptr_t)g.a & 15) == 0 &&
          ((uintptr_t)g.b & 15) == 0 && (g.epi == EPI_NONE || g.epi == EPI_BIAS) &&
          g.M / 16 < (1 << 30);
@@ -1384,8 +1398,8 @@ static bool f32_generic_better(const GemmArgs& g) {
 // that HIP takes (fewer than 2^32 threads in x, 256 per tile).
 static bool f32_mfma_ok(const GemmArgs& g) {
   constexpr int64_t kLim = (int64_t)1 << 30;
-  return g.dtype == REW_DT_FLOAT32 && g.c_dtype == REW_DT_FLOAT32 && g.K > 0 && g.M < kLim &&
-         g.N < kLim && g.K < kLim &&
+  return forced_tile() != 2 && g.dtype == REW_DT_FLOAT32 && g.c_dtype == REW_DT_FLOAT32 &&
+         g.K > 0 && g.M < kLim && g.N < kLim && g.K < kLim &&
          ((g.M + kFT - 1) / kFT) * ((g.N + kFT - 1) / kFT) * g.batch < (1 << 24) &&
          g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE && !f32_generic_better(g);
 }
@@ -1435,6 +1449,7 @@ static void launch_gemm_f32_mfma(const GemmArgs& g, hipStream_t stream) {
 //     10000 x 70: 239 / 345); otherwise no more (333 x 2816 x 1024: 178 / 71).
 static bool small_ok(const GemmArgs& g) {
   const int64_t tiles64 = ((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch;
+  if (forced_tile() == 2) return false;
   if (!f32_mfma_ok(g)) return tiles64 < 128 && g.epi != EPI_SWIGLU && g.epi != EPI_BIAS_ROPE;
   const int64_t tiles16 = ((g.M + 15) / 16) * ((g.N + 15) / 16) * g.batch;
   if (g.K > kSmallWholeK) {
@@ -1462,20 +1477,6 @@ static bool mfma_ok(const GemmArgs& g, bool* a_kc, bool* b_kc) {
   return true;
 }
 
-// The 256x256 kernel needs K-contiguous A and enough tiles to fill the
-// 256 CUs at least once; smaller problems run the 128x128 kernel.
-// REW_MI355X_GEMM_TILE=256 / 128 forces a kernel (tests use it to cover
-// the large-tile kernel's tails at small sizes); unset picks by size.
-// REW_MI355X_GEMM_TILE: "lds" (the direct-to-LDS kernels), "256" or "128".
-static int forced_tile() {
-  static const int v = [] {
-    const char* s = std::getenv("REW_MI355X_GEMM_TILE");
-    if (s && std::string(s) == "lds") return 1;
-    return s ? std::atoi(s) : 0;
-  }();
-  return v;
-}
-
 // The direct-to-LDS kernels run every bf16 GEMM they support once it has
 // enough 256x256 tiles to occupy most of the 256 CUs (or when forced).
 static bool use_lds(const GemmArgs& g) {
@@ -1499,6 +1500,8 @@ static bool epi256_ok(const GemmArgs& g) {
   return true;
 }
 
+// The 256x256 kernel needs K-contiguous A and enough tiles to fill the
+// 256 CUs at least once; smaller problems run the 128x128 kernel.
 static bool use_256(const GemmArgs& g, bool akc) {
   if (!akc || forced_tile() == 128 || !epi256_ok(g)) return false;
   const int64_t tiles = ((g.M + 255) / 256) * ((g.N + 255) / 256) * g.batch;
@@ -1527,10 +1530,11 @@ bool gemm_epilogue_ok(const GemmArgs& g) {
   return a_ext < (1ll << 31) && b_ext < (1ll << 31) && ((uintptr_t)g.b2 & 15) == 0;
 }
 
-const char* gemm_variant(const GemmArgs& g) {
+const char* gemm_variant(const GemmArgs* segs, bool multi, const StripPlan& strip) {
   bool akc, bkc;
-  if (gemm_strip_plan(&g, 1).R)
-    return g.epi == EPI_SWIGLU ? "gemm_lds_swiglu_strip" : "gemm_lds_nn_strip";
+  const GemmArgs& g = segs[0];
+  if (strip.R) return g.epi == EPI_SWIGLU ? "gemm_lds_swiglu_strip" : "gemm_lds_nn_strip";
+  if (multi) return g.epi == EPI_SWIGLU ? "gemm_lds_swiglu" : "gemm_lds_nn";
   if (use_lds(g)) {
     gemm_lds_ok(g, &bkc);
     return g.epi == EPI_SWIGLU ? "gemm_lds_swiglu" : (bkc ? "gemm_lds_tn" : "gemm_lds_nn");
@@ -1538,7 +1542,7 @@ const char* gemm_variant(const GemmArgs& g) {
   if (g.epi == EPI_SWIGLU) return "gemm_bf16_256_swiglu";
   if (!mfma_ok(g, &akc, &bkc))
     return f32_narrow_ok(g) ? "gemm_f32_narrow" : (small_ok(g) ? "gemm_f32_small"
-                                           : f32_mfma_ok(g) ? "gemm_generic_mfma" : "gemm_generic");
+                                           : f32_mfma_ok(g) ? "gemm_f32_mfma" : "gemm_generic");
   if (use_256(g, akc)) return bkc ? "gemm_bf16_256_tn" : "gemm_bf16_256_nn";
   if (akc && bkc) return "gemm_bf16_mfma_tn";
   if (akc) return "gemm_bf16_mfma_nn";

@@ -190,8 +190,8 @@ void launch_gemm_multi(const GemmArgs* segs, int n, const StripPlan& strip, hipS
 // Whether launch_gemm runs g with its epilogue (EPI_SWIGLU needs the large
 // dual kernel; the others run on every MFMA kernel).
 bool gemm_epilogue_ok(const GemmArgs& g);
-// Name of the kernel variant launch_gemm would pick (for profiles/tests).
-const char* gemm_variant(const GemmArgs& g);
+// Name of the kernel that launch_gemm or (multi) launch_gemm_multi picks.
+const char* gemm_variant(const GemmArgs* segs, bool multi, const StripPlan& strip);
 
 // ---- gather (k_gather.hip) ---------------------------------------------------
 // torch_index_select with batch_dims = 0: out[pre, i, post] =

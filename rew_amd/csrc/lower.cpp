@@ -1454,6 +1454,21 @@ void Lower::dot_args(Node* n, GemmArgs& g, Tensor*& ta_out, Tensor*& tb_out) {
   tb_out = tb;
 }
 
+// "<kernel><what>[batch,M,N,K]" (N of all segments): the shape fixes the
+// algorithmic FLOPs.  The strip kernel's row blocks and k splits follow.
+static std::string gemm_label(const GemmL& l, const std::string& what) {
+  const StripPlan p = gemm_strip_plan(l.g.data(), (int)l.g.size());
+  const GemmArgs& g = l.g[0];
+  long long n = 0;
+  for (const GemmArgs& s : l.g) n += s.N;
+  char nm[96];
+  std::snprintf(nm, sizeof nm, "[%lld,%lld,%lld,%lld]", (long long)g.batch, (long long)g.M, n,
+                (long long)g.K);
+  std::string name = gemm_variant(l.g.data(), l.multi, p) + what + nm;
+  if (p.R) name += " r" + std::to_string(p.R) + " s" + std::to_string(p.splits);
+  return name;
+}
+
 void Lower::emit_dot(Node* n) {
   auto fit = flash.find(n);
   if (fit != flash.end()) {
@@ -1475,13 +1490,7 @@ void Lower::emit_dot(Node* n) {
     run_launch(c, Launch{FillL{out->data(), nullptr, (size_t)out->nbytes()}});
   } else {
     Launch L{GemmL{{g}, false}};
-    if (c->profiling) {
-      // "<variant>[batch,M,N,K]": the shape fixes the algorithmic FLOPs
-      char nm[160];
-      std::snprintf(nm, sizeof nm, "%s[%lld,%lld,%lld,%lld]", gemm_variant(g),
-                    (long long)g.batch, (long long)g.M, (long long)g.N, (long long)g.K);
-      L.name = nm;
-    }
+    if (c->profiling) L.name = gemm_label(std::get<GemmL>(L.args), "");
     run_launch(c, std::move(L));
   }
   // canonical copies made for this GEMM die with it (stream-ordered free)
@@ -2083,23 +2092,15 @@ bool Lower::emit_gemm_fused(Tensor* t, const GemmPlan& p) {
       ok = gemm_fused_args(outs[i], plans[i], args[i]);
     if (ok) ok = gemm_multi_ok(args.data(), (int)args.size());
     if (ok) {
-      int64_t n_all = 0;
       std::string parts;
       for (size_t i = 0; i < outs.size(); ++i) {
         tensor_alloc(outs[i]);
         args[i].c = outs[i]->data();
-        n_all += args[i].N;
         parts += std::string(i ? "," : "") + std::to_string(args[i].N) + epi_suffix(args[i].epi);
         if (i) gemm_out.erase(outs[i]);
       }
       Launch L{GemmL{args, true}};
-      if (c->profiling) {
-        char nm[200];
-        std::snprintf(nm, sizeof nm, "%s{%s}[1,%lld,%lld,%lld]",
-                      p.epi == EPI_SWIGLU ? "gemm_lds_swiglu" : "gemm_lds_nn", parts.c_str(),
-                      (long long)args[0].M, (long long)n_all, (long long)args[0].K);
-        L.name = nm;
-      }
+      if (c->profiling) L.name = gemm_label(std::get<GemmL>(L.args), "{" + parts + "}");
       L.fused = true;
       run_launch(c, std::move(L));
       return true;
@@ -2116,13 +2117,7 @@ bool Lower::emit_gemm_fused(Tensor* t, const GemmPlan& p) {
   tensor_alloc(t);
   g.c = t->data();
   Launch L{GemmL{{g}, p.epi == EPI_BIAS_ROPE}};
-  if (c->profiling) {
-    char nm[160];
-    std::snprintf(nm, sizeof nm, "%s%s[%lld,%lld,%lld,%lld]",
-                  p.epi == EPI_BIAS_ROPE ? "gemm_lds_nn" : gemm_variant(g), epi_suffix(p.epi),
-                  (long long)g.batch, (long long)g.M, (long long)g.N, (long long)g.K);
-    L.name = nm;
-  }
+  if (c->profiling) L.name = gemm_label(std::get<GemmL>(L.args), epi_suffix(p.epi));
   L.fused = true;
   run_launch(c, std::move(L));
   return true;

@@ -11,6 +11,7 @@ pytestmark = pytest.mark.gpu
 
 from rew_amd import eager as E
 from rew_amd import nn
+from rew_amd import ops as O
 from rew_amd.eager import DType
 from test_gpu_attention import _expand, _qkv, _run, _sdpa_dir
 
@@ -43,6 +44,27 @@ def test_decode_matches_oracle(gpu, oracle, causal, B, H, Hkv, Sq, Sk, D):
     assert np.max(np.abs(got - want)) <= 1e-1 * np.max(np.abs(want))
     for _ in range(3):
         np.testing.assert_array_equal(_run(fn)[0], got)
+
+
+@pytest.mark.parametrize("Sk", [256, 300])
+def test_decode_over_a_longer_cache(gpu, oracle, Sk):
+    """Keys and values as the first Sk rows of a longer cache: the bits of dense
+    ones, and nothing of the rows behind."""
+    B, H, Hkv, Sq, D, S = 2, 8, 2, 2, 128, 512
+    q, k, v = _qkv(oracle, 3, B, H, Hkv, Sq, S, D)
+    qt = E.fromHost(q, DType.BFLOAT16)
+    k[:, :, Sk:], v[:, :, Sk:] = np.nan, np.inf
+
+    def fn(kt, vt):
+        return nn.scaledDotProductAttention(qt, _expand(kt, B, Hkv, 4, Sk, D),
+                                            _expand(vt, B, Hkv, 4, Sk, D))
+
+    cut = [O.slice_(E.fromHost(t, DType.BFLOAT16), [0, 0, 0, 0], [B, Hkv, Sk, D]) for t in (k, v)]
+    got, names = _run(lambda: fn(*cut))
+    assert any(n.startswith("flash_attn_dec") for n in names), names
+    dense = [E.fromHost(np.ascontiguousarray(t[:, :, :Sk]), DType.BFLOAT16) for t in (k, v)]
+    np.testing.assert_array_equal(got, _run(lambda: fn(*dense))[0])
+    assert np.all(np.isfinite(got))
 
 
 @pytest.mark.parametrize("direction,code", [("LE", 1), ("GE", 2), ("LT", 3), ("GT", 4)])

@@ -173,7 +173,7 @@ def test_llama_layer_kernel_plan(gpu, oracle):
     def launches(pred):
         return sum(cnt for n, cnt, _ in prof if pred(n))
 
-    assert launches(lambda n: n.startswith("gemm_lds_nn{") and n.count("+rope") == 2) == 1, names
+    assert launches(lambda n: n.startswith("gemm_lds_nn_strip{") and n.count("+rope") == 2) == 1, names
     assert launches(lambda n: n.startswith("rope_pairs")) == 0, names
     assert launches(lambda n: n.startswith("flash_attn")) == 1, names
     assert launches(lambda n: "swiglu" in n) == 1, names

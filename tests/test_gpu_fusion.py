@@ -427,7 +427,7 @@ def test_qkv_projections_one_launch(gpu, oracle, B, S, E_, H, KV, D):
         return res, names
 
     got, names = run(False)
-    assert any(n.startswith("gemm_lds_nn{") and n.count("+rope") == 2 for n in names), names
+    assert any(n.startswith("gemm_lds_nn_strip{") and n.count("+rope") == 2 for n in names), names
     ref, _ = run(True)
     for g_, r_ in zip(got, ref):
         np.testing.assert_array_equal(g_, r_)

@@ -1,6 +1,7 @@
 """GPU parity of the f32 matrix-core GEMM (gemm_f32_mfma_kernel).  Each output
-is the fmaf chain over k that the 16 x 16 kernel runs, so a slice of a
-product, small enough for that kernel, has the same bits as the product's."""
+is the fmaf chain over k that the generic and the 16 x 16 kernels run, so a
+slice of a product, small enough for the latter, has the same bits as the
+product's; the generic kernel's own bits come from a process that forces it."""
 import numpy as np
 import pytest
 
@@ -42,7 +43,7 @@ def test_chain_equals_small_kernel(gpu, oracle, form, M, K, N):
     a[3, 0], b[0, 5] = np.inf, np.nan
     _, f = FORMS[form]
     got, names = run(lambda: f(a, b))
-    assert any(n.startswith("gemm_generic_mfma") for n in names), names
+    assert any(n.startswith("gemm_f32_mfma") for n in names), names
     for m0, n0 in ((0, 0), (M - 33, N - 65), (M // 2, N // 3)):
         ref, names = run(lambda: f(a[m0:m0 + 33], b[:, n0:n0 + 65]))
         assert any(n.startswith("gemm_f32_small") for n in names), names
@@ -61,7 +62,7 @@ def test_batches_and_epilogues(gpu):
     B, M, K, N = 6, 333, 65, 331
     a, b = r.standard_normal((B, M, K)), r.standard_normal((B, K, N))
     got, names = run(lambda: O.dotGeneral(dev(a), dev(b), [0], [0], [2], [1]))
-    assert any(n.startswith("gemm_generic_mfma") for n in names), names
+    assert any(n.startswith("gemm_f32_mfma") for n in names), names
     a32, b32 = a.astype(np.float32), b.astype(np.float32)
     want = np.matmul(a32.astype(np.float64), b32.astype(np.float64))
     bound = (K + 1) * 2.0 ** -24 * np.matmul(np.abs(a32).astype(np.float64), np.abs(b32))
@@ -77,7 +78,7 @@ def test_batches_and_epilogues(gpu):
     for fn, ref in ((lin, plain + bias), (lambda: O.add(dev(res), lin()), res + (plain + bias)),
                     (lambda: nn.relu(lin()), np.maximum(plain + bias, 0))):
         out, names = run(fn)
-        assert len(names) == 1 and names[0].startswith("gemm_generic_mfma+bias"), names
+        assert len(names) == 1 and names[0].startswith("gemm_f32_mfma+bias"), names
         np.testing.assert_array_equal(out, ref)
 
 
@@ -97,10 +98,10 @@ def test_batch_past_the_grid_limit(gpu, M, K, N):
 
 @pytest.mark.parametrize("M,K,N,kernel", [
     (1, 1, 1, "gemm_generic"), (64, 7, 1, "gemm_generic"), (1, 7, 64, "gemm_generic"),
-    (3, 8, 3, "gemm_generic"), (2, 33, 2, "gemm_generic"), (13, 16, 13, "gemm_generic_mfma"),
-    (13, 15, 13, "gemm_generic"), (13, 17, 13, "gemm_generic_mfma"),
-    (8, 8, 8, "gemm_generic_mfma"), (65, 7, 3, "gemm_generic_mfma"),
-    (64, 8, 64, "gemm_generic_mfma"),
+    (3, 8, 3, "gemm_generic"), (2, 33, 2, "gemm_generic"), (13, 16, 13, "gemm_f32_mfma"),
+    (13, 15, 13, "gemm_generic"), (13, 17, 13, "gemm_f32_mfma"),
+    (8, 8, 8, "gemm_f32_mfma"), (65, 7, 3, "gemm_f32_mfma"),
+    (64, 8, 64, "gemm_f32_mfma"),
 ])
 def test_batches_of_small_products(gpu, M, K, N, kernel):
     """Which kernel takes 1500 products of one tile each, and its sums."""
@@ -125,7 +126,7 @@ def test_one_row_tile_keeps_its_height(gpu):
             E.flush()
             prof = E.profileEnd()
             del out
-            assert len(prof) == 1 and prof[0][0].startswith("gemm_generic_mfma"), prof
+            assert len(prof) == 1 and prof[0][0].startswith("gemm_f32_mfma"), prof
             best = min(best, prof[0][2] * 1e3)
         return best
 
@@ -136,10 +137,10 @@ def test_one_row_tile_keeps_its_height(gpu):
 
 @pytest.mark.parametrize("M,K,N,kernel", [
     (8, 1024, 2816, "gemm_f32_small"), (16, 1024, 4096, "gemm_f32_small"),
-    (17, 1024, 4096, "gemm_generic_mfma"), (32, 512, 4096, "gemm_f32_small"),
-    (33, 512, 4096, "gemm_generic_mfma"), (1, 4096, 4096, "gemm_f32_small"),
-    (8, 2048, 1024, "gemm_f32_small"), (9, 2048, 1024, "gemm_generic_mfma"),
-    (100, 3000, 70, "gemm_f32_small"), (100, 3000, 72, "gemm_generic_mfma"),
+    (17, 1024, 4096, "gemm_f32_mfma"), (32, 512, 4096, "gemm_f32_small"),
+    (33, 512, 4096, "gemm_f32_mfma"), (1, 4096, 4096, "gemm_f32_small"),
+    (8, 2048, 1024, "gemm_f32_small"), (9, 2048, 1024, "gemm_f32_mfma"),
+    (100, 3000, 70, "gemm_f32_small"), (100, 3000, 72, "gemm_f32_mfma"),
 ])
 def test_few_rows(gpu, M, K, N, kernel):
     """Which kernel takes a product of few rows, and its sums."""
@@ -162,9 +163,60 @@ def test_products_that_underflow(gpu, form, K):
     b = np.full((K, 648), 1e-20, np.float32)
     b[:, ::2] = 1e-30  # (the products underflow)
     got, names = run(lambda: f(a, b))
-    assert any(n.startswith("gemm_generic_mfma") for n in names), names
+    assert any(n.startswith("gemm_f32_mfma") for n in names), names
     ref, names = run(lambda: f(a[:33], b[:, :65]))
     assert any(n.startswith("gemm_f32_small") for n in names), names
     np.testing.assert_array_equal(got[:33, :65].view(np.uint32), ref.view(np.uint32))
     assert (ref[0, 0] == 0) and np.signbit(ref[0, 0]) == (K % 16 == 0)
     assert 0 < -ref[0, 1] < 1e-37
+
+
+GENERIC_CHILD = r"""
+import sys
+import numpy as np
+sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+from test_gpu_gemm_f32 import FORMS, generic_cases, run
+from rew_amd import eager as E
+E.installEagerBackend(E.mi355x(0))
+out = []
+for form, a, b in generic_cases():
+    got, names = run(lambda: FORMS[form][1](a, b))
+    assert [n.split("[")[0] for n in names] == ["gemm_generic"], names
+    out.append(got)
+np.savez(sys.argv[2], *out)
+"""
+
+
+def generic_cases():
+    r = np.random.default_rng(6)
+    for M, K, N in ((577, 100, 641), (640, 48, 644), (1100, 33, 8260), (64, 200, 70), (16, 64, 16),
+                    (300, 128, 32), (8, 2100, 300)):
+        for form in ("nn", "tt"):
+            a = r.standard_normal((M, K)).astype(np.float32)
+            b = (r.standard_normal((K, N)) * 10.0 ** r.integers(-3, 3, (K, N))).astype(np.float32)
+            a[:, K // 2:] *= np.float32(1e-25)
+            b[:, 1::3] *= np.float32(1e-16)  # sums of denormals in between
+            a[3] = 1e-30
+            b[:, 0] = -1e-30                 # products that underflow
+            yield form, a, b
+
+
+def test_equals_the_generic_kernel(gpu, tmp_path):
+    """The matrix-core, 16 x 16, 8 x 8 and narrow kernels against the generic one."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    out = str(tmp_path / "generic.npz")
+    p = subprocess.run([sys.executable, "-c", GENERIC_CHILD,
+                        str(Path(__file__).resolve().parents[1]), out],
+                       env=dict(os.environ, REW_MI355X_GEMM_TILE="generic"),
+                       capture_output=True, text=True, timeout=90)
+    assert p.returncode == 0, p.stderr[-3000:]
+    ref = np.load(out)
+    seen = set()
+    for i, (form, a, b) in enumerate(generic_cases()):
+        got, names = run(lambda: FORMS[form][1](a, b))
+        seen |= {n.split("[")[0] for n in names}
+        np.testing.assert_array_equal(got.view(np.uint32), ref[f"arr_{i}"].view(np.uint32))
+    assert seen == {"gemm_f32_mfma", "gemm_f32_small", "gemm_f32_narrow"}, seen

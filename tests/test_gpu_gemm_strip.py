@@ -26,17 +26,30 @@ def _dev(a):
     return E.fromHost(a, DType.BFLOAT16)
 
 
-@pytest.mark.parametrize("M,K,N", [
-    (1, 64, 8),          # one row, one k-tile, fewer columns than a wave
-    (32, 8, 128),        # K below a k-tile; exactly one tile
-    (33, 136, 264),      # a second row block, K and N remainders
-    (64, 1000, 392),     # partial last k-tile with 16 of them
-    (160, 192, 1032),    # five row blocks
-    (161, 2048, 520),    # split sums with a ragged second row tile
-    (8, 14336, 256),     # the deepest split
-    (129, 1032, 136),    # split, partial last k-tile in the last split only
-])
-def test_strip_linear_and_residual(gpu, M, K, N):
+# M, K, N, row blocks per tile, whether k is split
+LINEAR = [
+    (1, 64, 8, 1, False),          # one row, one k-tile, fewer columns than a wave
+    (32, 8, 128, 1, False),        # K below a k-tile; exactly one tile
+    (33, 136, 264, 1, False),      # a second row tile of one row, K and N remainders
+    (64, 1000, 392, 1, False),     # partial last k-tile with 16 of them
+    (161, 2048, 520, 1, True),     # split sums with a ragged last row tile
+    (8, 14336, 256, 1, True),      # the deepest split
+    (129, 1032, 136, 1, True),     # split, partial last k-tile in the last split only
+    (161, 72, 8200, 2, False),     # every number of row blocks: ragged last row tiles,
+    (33, 4104, 4104, 2, True),     # partial last k-tiles, N remainders
+    (700, 72, 5128, 4, False),
+    (97, 4104, 8200, 4, True),
+    (130, 4104, 8200, 5, True),
+]
+
+
+def _plan(name):
+    r, s = name.rsplit(" r", 1)[1].split(" s")
+    return int(r), int(s) > 1
+
+
+@pytest.mark.parametrize("M,K,N,R,split", LINEAR)
+def test_strip_linear_and_residual(gpu, M, K, N, R, split):
     r = np.random.default_rng(M * 7 + K + N)
     x, w, b = _bf16(r, (M, K), 1.0), _bf16(r, (K, N), 0.05), _bf16(r, (N,), 1.0)
     res = _bf16(r, (M, N), 1.0)
@@ -51,6 +64,7 @@ def test_strip_linear_and_residual(gpu, M, K, N):
         got = E.toHostF32(fn())
         names = [n for n, _, _ in E.profileEnd()]
         assert len(names) == 1 and names[0].startswith("gemm_lds_nn_strip+bias"), names
+        assert _plan(names[0]) == (R, split), names
         want = exact + b + (res if add else 0)
         size = np.abs(exact) + np.abs(b) + (np.abs(res) if add else 0)
         assert np.all(np.abs(got - want) <= 3 * 2.0 ** -8 * size + K * 2.0 ** -24 * mag)
@@ -58,21 +72,66 @@ def test_strip_linear_and_residual(gpu, M, K, N):
             np.testing.assert_array_equal(E.toHostF32(fn()), got)
 
 
-@pytest.mark.parametrize("T,H,I", [(1, 64, 8), (33, 136, 264), (40, 2048, 384), (150, 1032, 200)])
-def test_strip_swiglu(gpu, oracle, T, H, I):
+@pytest.mark.parametrize("T,H,I,R,split", [
+    (1, 64, 8, 1, False), (33, 136, 264, 1, False), (40, 2048, 384, 1, True),
+    (150, 1032, 200, 1, True), (161, 72, 8200, 2, False), (33, 2056, 5128, 2, True),
+    (97, 8200, 5128, 4, True), (130, 4104, 8200, 5, True),
+])
+def test_strip_swiglu(gpu, oracle, T, H, I, R, split):
+    """The gate and up products of every number of row blocks; a down projection
+    of 8 columns reads every element of theirs."""
+    rb = oracle.round_bf16
     r = np.random.default_rng(T + H + I)
     x = _bf16(r, (T, H), 1.0)
-    ws = [_bf16(r, s, 0.05) for s in ((H, I), (H, I), (I, H))]
-    bs = [_bf16(r, (n,), 0.5) for n in (I, I, H)]
+    ws = [_bf16(r, s, 0.02) for s in ((H, I), (H, I), (I, 8))]
+    bs = [_bf16(r, (n,), 0.5) for n in (I, I, 8)]
     ffn = nn.GatedFeedForward(*[nn.Linear(_dev(w), _dev(b)) for w, b in zip(ws, bs)])
+    xt = _dev(x.reshape(1, T, H))
     E.profileBegin()
-    got = E.toHostF32(ffn.forward(_dev(x.reshape(1, T, H)))).reshape(T, H)
+    got = E.toHostF32(ffn.forward(xt)).reshape(T, 8)
     names = [n for n, _, _ in E.profileEnd()]
-    assert any(n.startswith("gemm_lds_swiglu_strip") for n in names), names
-    want = oracle.gated_ffn(x, ws[0], bs[0], ws[1], bs[1], ws[2], bs[2], True)
-    # the oracle rounds where the op sequence does; sums in another order move
-    # a rounding of the hidden row by one bf16 ulp now and then
-    assert np.linalg.norm(got - want) <= 2e-3 * np.linalg.norm(want)
+    dual = [n for n in names if n.startswith("gemm_lds_swiglu_strip")]
+    assert len(dual) == 1 and _plan(dual[0]) == (R, split), names
+    f = lambda y, i: rb(rb((y.astype(np.float64) @ ws[i]).astype(np.float32)) + bs[i])  # noqa: E731
+    gate, up = f(x, 0), f(x, 1)
+    want = f(rb(gate * (np.float32(1) / (np.float32(1) + np.exp(-gate))) * up), 2)
+    # two roundings to bf16 behind the sums, and roundings of the hidden row
+    # that sums in another order move by one bf16 ulp now and then
+    assert np.all(np.linalg.norm(got - want, axis=0) <= 4e-3 * np.linalg.norm(want, axis=0))
+    for _ in range(3):
+        np.testing.assert_array_equal(E.toHostF32(ffn.forward(xt)).reshape(T, 8), got)
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 136, 264), (161, 2048, 520), (33, 4104, 4104)])
+def test_strip_views(gpu, M, K, N):
+    """Rows of a wider matrix times columns of a wider weight: the bits of dense ones."""
+    r = np.random.default_rng(M + K)
+    x, w = _bf16(r, (M, K + 24), 1.0), _bf16(r, (K, N + 40), 0.05)
+    E.profileBegin()
+    got = E.toHost(O.matmul(O.slice_(_dev(x), [0, 16], [M, 16 + K]),
+                            O.slice_(_dev(w), [0, 32], [K, 32 + N])))
+    names = [n for n, _, _ in E.profileEnd()]
+    assert any("_strip[" in n for n in names), names
+    want = E.toHost(O.matmul(_dev(np.ascontiguousarray(x[:, 16:16 + K])),
+                             _dev(np.ascontiguousarray(w[:, 32:32 + N]))))
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 136, 264), (161, 2048, 520), (129, 1032, 136)])
+def test_strip_infinities(gpu, M, K, N):
+    """Infinities and NaN reach their row and column and nothing else, past the
+    partial last k-tile and through the split sums."""
+    r = np.random.default_rng(M + N)
+    x, w = _bf16(r, (M, K), 1.0), _bf16(r, (K, N), 0.05)
+    clean = E.toHostF32(O.matmul(_dev(x), _dev(w)))
+    x[3, 5], x[M - 1, K - 1], w[7, 9], w[K - 1, N - 1] = np.inf, -np.inf, np.nan, np.inf
+    got = E.toHostF32(O.matmul(_dev(x), _dev(w)))
+    with np.errstate(invalid="ignore"):
+        want = (x.astype(np.float64) @ w.astype(np.float64)).astype(np.float32)
+    odd = ~np.isfinite(want)
+    np.testing.assert_array_equal(got[odd], want[odd])
+    np.testing.assert_array_equal(got[~odd], clean[~odd])
+    assert odd.sum() == 2 * (M + N) - 4
 
 
 @pytest.mark.parametrize("B,S", [(1, 1), (2, 33)])
@@ -97,7 +156,8 @@ def test_strip_projections_with_rope(gpu, oracle, B, S):
     E.profileBegin()
     outs = [E.toHostF32(t) for t in fn()]
     names = [n for n, _, _ in E.profileEnd()]
-    assert any(n.startswith("gemm_lds_nn{") and n.count("+rope") == 2 for n in names), names
+    sets = [n for n in names if n.startswith("gemm_lds_nn_strip{") and n.count("+rope") == 2]
+    assert len(sets) == 1 and _plan(sets[0]) == (1, True), names
     for got, (w, b), n, rot in zip(outs, lin, (nh, nkv, nkv), (True, True, False)):
         y = oracle.round_bf16(oracle.round_bf16((x.astype(np.float64) @ w).astype(np.float32)) + b)
         y = y.reshape(B, S, n, hd).transpose(0, 2, 1, 3)

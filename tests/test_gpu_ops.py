@@ -239,12 +239,12 @@ def test_matmul_f32_narrow(gpu, oracle, M, K, N):
                                    # its limit
                                    (37, 100, 72), (130, 52, 20), (16, 12, 8),
                                    (72, 1024, 68)])
-def test_matmul_f32_small_equals_generic(gpu, oracle, M, K, N):
+def test_matmul_f32_small_equals_matrix_core_batch(gpu, oracle, M, K, N):
     """Products with too few 64x64 tiles to fill the GPU (the MNIST MLP's)
     take 16x16 tiles, or one wave per 8x8 tile when even the 16x16 tiles
-    would leave most CUs idle; each output keeps the generic kernel's fmaf
+    would leave most CUs idle; each output keeps the other kernels' fmaf
     chain, so a batch of 128 of the same product (enough tiles for the
-    generic kernel) gives the same bits in every slice."""
+    matrix-core kernel) gives the same bits in every slice."""
     r = rng(M * 3 + K + N)
     a = r.uniform(-1, 1, (M, K)).astype(np.float32)
     b = r.uniform(-0.1, 0.1, (K, N)).astype(np.float32)
@@ -257,7 +257,7 @@ def test_matmul_f32_small_equals_generic(gpu, oracle, M, K, N):
     E.profileBegin()
     ref = host(O.dotGeneral(dev(ab), dev(bb), [0], [0], [2], [1]))
     names = [n for n, _, _ in E.profileEnd()]
-    assert any(n.startswith("gemm_generic") for n in names), names
+    assert any(n.startswith("gemm_f32_mfma") for n in names), names
     for i in range(128):
         np.testing.assert_array_equal(ref[i].view(np.uint32), got.view(np.uint32))
     bound = 1e-5 * oracle.gemm(np.abs(a), np.abs(b))
