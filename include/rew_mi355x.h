@@ -250,10 +250,10 @@ int rew_mi355x_profile_entry(rew_mi355x_ctx* ctx, int index, char* name,
                              int name_cap, int64_t* launches, double* total_ms);
 
 /* Native stream of the context (a hipStream_t), for callers that record
- * their own events around the backend's work.  Split products and decode
- * attention keep partial results in one array per GPU, ordered by this
- * stream: launches captured from it must not be replayed on another stream
- * while it has work. */
+ * their own events around the backend's work.  Launches captured from it into
+ * a graph share no working memory with later ones: products and decode
+ * attention that split their sums over workgroups otherwise do not when
+ * captured, so their results may differ in the last rounding. */
 int rew_mi355x_stream(rew_mi355x_ctx* ctx, void** out_stream);
 
 /* ---- routed mixture-of-experts FFN over caller-owned device rows ---------

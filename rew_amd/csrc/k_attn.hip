@@ -1000,8 +1000,8 @@ constexpr int kDecMaxPairs = 4096;
 constexpr int64_t kDecWs = 4ll << 20;  // floats: partial O, then (max, sum) pairs
 constexpr int kAgent = 16;             // cache policy sc1: agent-scope access
 }  // namespace fa
-// (all launches of a device are ordered on its context's stream, and each
-// leaves the counts at zero)
+// (all launches of a device are ordered on its context's stream, each leaves the
+// counts at zero, and captured ones are not split)
 __device__ float g_dec_o[fa::kDecWs];
 __device__ float g_dec_ml[fa::kDecWs / 16];
 __device__ int g_dec_count[fa::kDecMaxPairs];
@@ -1326,11 +1326,11 @@ static bool flash_dec_ok(const FlashArgs& a) {
 // Key tiles per split: the fewest rounds of tiles over the CUs (two waves a
 // workgroup; at D = 128 one workgroup a CU, else two), a merge counted as one
 // more and another for each eight columns it reads.
-static void flash_dec_plan(const FlashArgs& a, int* splits, int* per) {
+static void flash_dec_plan(const FlashArgs& a, int max_splits, int* splits, int* per) {
   const int64_t pairs = (int64_t)a.B * a.Hkv, rows = (int64_t)(a.H / a.Hkv) * a.Sq;
   const int64_t nkt = (a.Sk + fa::BKV - 1) / fa::BKV, slots = a.D == 128 ? 256 : 512;
   int64_t best = 1ll << 60;
-  for (int64_t s = 1; s <= 64 && s <= nkt; ++s) {
+  for (int64_t s = 1; s <= max_splits && s <= nkt; ++s) {
     if (s > 1 && (pairs > fa::kDecMaxPairs || pairs * s * rows * a.D > fa::kDecWs ||
                   pairs * s * rows * 2 > fa::kDecWs / 16))
       break;
@@ -1368,7 +1368,8 @@ void launch_flash(const FlashArgs& a, hipStream_t stream) {
     // (at most 32 queries: where they see no key past their own, one tile is all)
     FlashArgs d = a;
     if (hides_past_diagonal(a)) d.Sk = std::min(a.Sk, fa::BKV);
-    flash_dec_plan(d, &splits, &per);
+    flash_dec_plan(d, 64, &splits, &per);
+    if (splits > 1 && being_captured(stream)) flash_dec_plan(d, 1, &splits, &per);
     const unsigned grid = (unsigned)(a.B * a.Hkv * splits);
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(grid), dim3(128), 0, stream, d, splits, per);

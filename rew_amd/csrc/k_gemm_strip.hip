@@ -77,8 +77,8 @@ __device__ __forceinline__ void block_barrier() {
 
 // Partial tiles of split products and the arrivals per tile.  All launches
 // of a device's context are ordered on its one stream and each leaves the
-// counters at zero, so one array per device serves every launch; work that
-// replays captured launches on another stream meanwhile would race with it.
+// counters at zero, so one array per device serves every launch (captured ones,
+// which may run beside that stream, are not split).
 constexpr int64_t kWsFloats = 12ll << 20;  // 48 MiB
 constexpr int kMaxSplitTiles = 1024;
 constexpr int kAgent = 16;  // cache policy sc1: agent-scope access
@@ -448,7 +448,7 @@ int64_t col_tiles(const GemmArgs& g) { return (g.N + BN - 1) / BN; }
 //   * 4 us around them.
 // K below 1024 is never split: there is little to gain, and the sum then
 // runs in the order of the 256 x 256 kernel's.
-StripPlan plan_for(const GemmArgs* segs, int n) {
+StripPlan plan_for(const GemmArgs* segs, int n, int max_splits) {
   const int64_t M = segs[0].M, K = segs[0].K;
   const bool dual = segs[0].epi == EPI_SWIGLU;
   const int64_t nk = (K + BK - 1) / BK;
@@ -465,7 +465,7 @@ StripPlan plan_for(const GemmArgs* segs, int n) {
   for (int x = 0; x < 4; ++x) {
     const int64_t tm = (M + 32 * kR[x] - 1) / (32 * kR[x]), tiles = tm * best.tiles_n;
     const int64_t fit = kWsFloats / (tiles * 32 * kR[x] * BN * (dual ? 2 : 1));
-    for (int64_t s = 1; s <= 16; ++s) {
+    for (int64_t s = 1; s <= max_splits; ++s) {
       if (s > 1 && (K < 1024 || s > nk / 8 || s > fit || tiles > kMaxSplitTiles)) break;
       const int64_t per = (nk + s - 1) / s, wgs = tiles * s;
       const double fill = wgs > 256 ? (double)wgs / 256 : 1.0;
@@ -522,7 +522,7 @@ void go(const GemmSegs& gs, const StripPlan& p, hipStream_t stream) {
 
 }  // namespace
 
-StripPlan gemm_strip_plan(const GemmArgs* segs, int n) {
+StripPlan gemm_strip_plan(const GemmArgs* segs, int n, int max_splits) {
   const StripPlan none;
   static const bool forced = std::getenv("REW_MI355X_GEMM_TILE") != nullptr;
   if (forced || n < 1 || n > kMaxSegs) return none;
@@ -547,7 +547,7 @@ StripPlan gemm_strip_plan(const GemmArgs* segs, int n) {
   // kernel or, as SwiGLU, to the older 256 x 256 one, which no size measured had
   // faster (8 x 14336 x 4096: 443 us against 28 here; SwiGLU 1500 x 2048 x 1408:
   // 92 against 49).
-  const StripPlan p = plan_for(segs, n);
+  const StripPlan p = plan_for(segs, n, max_splits);
   if (tiles < 96 && n == 1) return p;
   // From there on the two estimates decide, where they differ by more than
   // their bias: the 256 x 256 kernel had every product of more than 256 rows
@@ -560,6 +560,12 @@ StripPlan gemm_strip_plan(const GemmArgs* segs, int n) {
   const double here = strip_time(p, f.K, weights, dual);
   const double there = tile256_time(tiles, f.K, weights, dual);
   return here < (dual && f.M > 64 ? 0.85 : 0.97) * there ? p : none;
+}
+
+bool being_captured(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  REW_HIP(hipStreamIsCapturing(stream, &st));
+  return st != hipStreamCaptureStatusNone;
 }
 
 void launch_gemm_strip(const GemmArgs* segs, int n, const StripPlan& p, hipStream_t stream) {

@@ -120,7 +120,13 @@ struct StripPlan {
 };
 // The plan depends on shapes, strides and alignments alone, so a recorded
 // launch keeps it.
-StripPlan gemm_strip_plan(const GemmArgs* segs, int n);
+constexpr int kMaxStripSplits = 16;
+StripPlan gemm_strip_plan(const GemmArgs* segs, int n, int max_splits = kMaxStripSplits);
+// Whether what is launched on `stream` is being captured into a graph.  The
+// partial results of split products and split decode attention lie in one
+// array per GPU, in the order of the context's stream; a captured launch may
+// be replayed on another stream beside it, so it is not split.
+bool being_captured(hipStream_t stream);
 void launch_gemm_strip(const GemmArgs* segs, int n, const StripPlan& plan, hipStream_t stream);
 
 // strip: gemm_strip_plan's answer for g.

@@ -183,8 +183,11 @@ struct Exec {
       l.strip = gemm_strip_plan(l.g.data(), (int)l.g.size());
       l.planned = true;
     }
-    if (l.multi) launch_gemm_multi(l.g.data(), (int)l.g.size(), l.strip, c->stream);
-    else launch_gemm(l.g[0], l.strip, c->stream);
+    const StripPlan strip = l.strip.splits > 1 && being_captured(c->stream)
+                                ? gemm_strip_plan(l.g.data(), (int)l.g.size(), 1)
+                                : l.strip;
+    if (l.multi) launch_gemm_multi(l.g.data(), (int)l.g.size(), strip, c->stream);
+    else launch_gemm(l.g[0], strip, c->stream);
   }
   void operator()(FlashArgs& a) { launch_flash(a, c->stream); }
   void operator()(RowNormArgs& a) { launch_rmsnorm_rows(a, c->stream); }
