@@ -122,7 +122,7 @@ def test_swiglu_gate_and_up_far_apart(gpu, oracle):
         return ffn.forward(E.fromHost(x, DType.BFLOAT16))
 
     got, names = _run(fn)
-    assert any(n.startswith("gemm_lds_swiglu") for n in names), names
+    assert any(n.startswith("gemm_lds_swiglu[") for n in names), names
     ref, _ = _run(fn, op_by_op=True)
     np.testing.assert_array_equal(got, ref)
     want = oracle.gated_ffn(x.reshape(T, E_), wg, bg, wu, bu, wd, bd, True).reshape(1, T, E_)

@@ -165,6 +165,55 @@ def test_strip_projections_with_rope(gpu, oracle, B, S):
         assert np.linalg.norm(got - want) <= 4e-3 * np.linalg.norm(want)
 
 
+ROPE_CHILD = r"""
+import sys
+import numpy as np
+sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+from test_gpu_gemm_strip import rope_sets
+from rew_amd import eager as E
+E.installEagerBackend(E.mi355x(0))
+np.savez(sys.argv[2], *rope_sets("gemm_lds_nn{"))
+"""
+
+
+def rope_sets(label):
+    """q / k / v projections with ragged row and column tiles of either kernel."""
+    r = np.random.default_rng(12)
+    res = []
+    for B, S, nh, nkv, hd, H in ((2, 33, 3, 1, 24, 136), (1, 300, 5, 2, 72, 264)):
+        x = _dev(_bf16(r, (B * S, H), 1.0))
+        rope = nn.RotaryPositionEncoding.init(hd, S, 10000.0)
+        outs = []
+        E.profileBegin()
+        for n, rot in ((nh, True), (nkv, True), (nkv, False)):
+            w, b = _bf16(r, (H, n * hd), 0.05), _bf16(r, (n * hd,), 0.2)
+            y = O.reshape(nn.Linear(_dev(w), _dev(b)).forward(x), [B, S, n, hd])
+            y = O.transpose(y, [0, 2, 1, 3])
+            outs.append(rope.forward(y) if rot else O.add(y, y))
+        E.flush()
+        names = [n for n, _, _ in E.profileEnd()]
+        assert any(n.startswith(label) and n.count("+rope") == 2 for n in names), names
+        res += [E.toHostF32(t) for t in outs]
+    return res
+
+
+def test_rope_sets_equal_the_256_tiles(gpu, tmp_path):
+    """Unsplit sets on both kernels: the same sums in the same order."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    out = str(tmp_path / "sets.npz")
+    p = subprocess.run([sys.executable, "-c", ROPE_CHILD,
+                        str(Path(__file__).resolve().parents[1]), out],
+                       env=dict(os.environ, REW_MI355X_GEMM_TILE="lds"), capture_output=True,
+                       text=True, timeout=90)
+    assert p.returncode == 0, p.stderr[-3000:]
+    ref = np.load(out)
+    for i, got in enumerate(rope_sets("gemm_lds_nn_strip{")):
+        np.testing.assert_array_equal(got, ref[f"arr_{i}"])
+
+
 def test_reversed_rows(gpu):
     """A view with a negative row stride takes none of the kernels that form
     unsigned offsets from the view's base."""

@@ -142,7 +142,8 @@ def test_moe_sparse_equals_dense_op_by_op(gpu, oracle):
 def test_moe_few_tokens(gpu, oracle, T, H, I, n_shared):
     """Up to 128 tokens every group takes 64-row tiles, by a kernel of their
     own; each output keeps its MFMA sequence, so the values equal the dense
-    op-by-op ones (129 tokens and I 136 take the other kernels)."""
+    op-by-op ones, whose products are not split below K 1024 (129 tokens and I
+    136 take the other kernels)."""
     moe, host = build_moe(oracle, T, H, I, 8, 2, n_shared, 0x5EED0505 + T)
     xt = E.fromHost(host["x"], DType.BFLOAT16)
     sparse = E.toHostF32(moe.forward(xt))
@@ -152,6 +153,29 @@ def test_moe_few_tokens(gpu, oracle, T, H, I, n_shared):
     finally:
         E.setMode(E.MODE_DEFERRED)
     np.testing.assert_array_equal(sparse, dense)
+
+
+@pytest.mark.parametrize("T,H,I", [(40, 1024, 1032), (8, 2048, 1408)])
+def test_moe_few_tokens_against_split_products(gpu, oracle, T, H, I):
+    """From K 1024 on the dense Linears of few tokens split their sums over
+    workgroups, and the grouped products do not: the values differ by roundings.
+    Of a bf16 value's roundings about one in a thousand falls the other way when
+    its sum of K terms moves by some sqrt(K) 2^-24, a step of up to 2^-7; with the
+    dozen roundings behind each output that is sqrt(0.012) 2^-7 = 9e-4 of the
+    norm, and no element moves by more than a dozen steps."""
+    moe, host = build_moe(oracle, T, H, I, 8, 2, 2, 0x5EED0515 + T)
+    xt = E.fromHost(host["x"], DType.BFLOAT16)
+    sparse = E.toHostF32(moe.forward(xt))
+    E.setMode(E.MODE_OP_BY_OP)
+    try:
+        E.profileBegin()
+        dense = E.toHostF32(moe.forward(xt))
+        names = [n for n, _, _ in E.profileEnd()]
+    finally:
+        E.setMode(E.MODE_DEFERRED)
+    assert any("_strip" in n and int(n.rsplit(" s", 1)[1]) > 1 for n in names), names
+    assert np.linalg.norm(sparse - dense) <= 1e-3 * np.linalg.norm(dense)
+    assert np.max(np.abs(sparse - dense)) <= 12 * 2.0 ** -7 * np.max(np.abs(dense))
 
 
 def small_and_large_groups(oracle):
@@ -234,7 +258,8 @@ def test_moe_expert_matrices_far_apart(gpu, oracle):
     expert 5's through the C-ABI entry point: the grouped GEMM does the same
     for every expert.  Same bits as with the weights near each other."""
     from test_gpu_fusion import far_apart
-    moe, host = build_moe(oracle, 512, 256, 128, 16, 4, 2, 0x5EED0905)
+    # (tokens enough that the shared pair takes the 256-row tiles)
+    moe, host = build_moe(oracle, 4096, 256, 512, 16, 4, 2, 0x5EED0905)
     xt = E.fromHost(host["x"], DType.BFLOAT16)
     near = E.toHost(moe.forward(xt))
     sh = host["shared"][1]
@@ -255,7 +280,7 @@ def test_moe_expert_matrices_far_apart(gpu, oracle):
     prof = [n for n, _, _ in E.profileEnd()]
     # (weights seen through pending views stay out of the MoE group: the two
     # shared SwiGLU GEMMs run as their own two-segment launch)
-    assert any(n.startswith("gemm_lds_swiglu{128,128}") for n in prof), prof
+    assert any(n.startswith("gemm_lds_swiglu{512,512}") for n in prof), prof
     np.testing.assert_array_equal(far, near)
 
     # the routed grouped GEMM: expert 5's up weight read 2 GiB past a copy
