@@ -185,9 +185,10 @@ __device__ __forceinline__ void tile_order(int64_t bid, int64_t tiles_m, int64_t
 // runs.  Its A stages are a quarter as tall, the LDS comes to 80 KiB and two
 // workgroups share a CU: the weight stream is what bounds such a launch, and
 // twice the bytes are in flight while one tile's prologue or epilogue runs.
-// 40 tokens over 64 + 2 experts of 2048 x 1408, the whole block: 277.7 ->
-// 271.3 us (on boxes where one earlier build took 296.1 and 294.6).  Above
-// kSmallGroupRows tokens a group may need 256-row tiles.
+// 64 + 2 experts of 2048 x 1408, the block's launches with and without, in turn
+// on one box: 16 tokens 249 us / 265, 40 274 / 278, 64 294 / 302, 128 297 / 305;
+// 1 and 4 tokens within the spread.  Above kSmallGroupRows tokens a group may
+// need 256-row tiles.
 template <bool B_KC, bool DUAL, bool GROUP, bool BUF, bool FAR = false, bool LOW = false>
 __global__ void __launch_bounds__(256, LOW ? 2 : 1) gemm_lds_kernel(GemmSegs gs, GroupArgs ga) {
   static_assert(!LOW || (GROUP && BUF && !B_KC), "64-row tiles: grouped buffer path");
