@@ -148,16 +148,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t fa_rsrc(const void* base,
 struct FaRows {
   const uint16_t* p;
   int64_t step;
-  int left;  // bytes from p to the end of the last row
+  uint32_t left;  // bytes from p to the end of the last row (any, past it)
   __device__ __forceinline__ FaRows(const uint16_t* base, int k0, int rows, int64_t stride, int D,
                                     int step_rows)
       : p(base + k0 * stride), step(step_rows * stride),
-        left((int)(((rows - 1 - k0) * stride + D) * 2)) {}
+        left((uint32_t)(((rows - 1 - k0) * stride + D) * 2)) {}
   // the descriptor of this tile (none of it unless live), and on to the next
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t next(bool live) {
-    const __amdgpu_buffer_rsrc_t r = fa_rsrc(p, live ? (uint32_t)left : 0u);
+    const __amdgpu_buffer_rsrc_t r = fa_rsrc(p, live ? left : 0u);
     p += step;
-    left -= (int)step * 2;
+    left -= (uint32_t)step * 2;
     return r;
   }
 };
@@ -992,8 +992,8 @@ __global__ void __launch_bounds__(512, 1) flash_pp_kernel(FlashArgs a) {
 // A wave's running max, sum and O (fp32) join the other wave's through LDS;
 // the workgroups' go to memory past the L2 (agent scope) and the last to
 // arrive merges them in split order, as in the strip GEMM.
-// 16 x 32 / 8 heads x 4000 keys x 128 (262 MB of K and V): 130 -> 54 us
-// (4.9 TB/s).
+// 16 x 32 / 8 heads x 4000 keys x 128 (262 MB of K and V): 127 -> 52 us
+// (5.0 TB/s).
 namespace fa {
 constexpr int kDecCols = 32;
 constexpr int kDecMaxPairs = 4096;
@@ -1296,9 +1296,11 @@ static int flash_forced() {
   return v;
 }
 
+// (a tile's offsets run to its 64th row, whether or not there is one)
 static bool flash_buf_ok(const FlashArgs& a) {
-  return a.k_ss >= 0 && a.v_ss >= 0 && ((int64_t)a.Sk * a.k_ss + a.D) * 2 < (1ll << 31) &&
-         ((int64_t)a.Sk * a.v_ss + a.D) * 2 < (1ll << 31);
+  const int64_t rows = std::max(a.Sk, fa::BKV);
+  return a.k_ss >= 0 && a.v_ss >= 0 && (rows * a.k_ss + a.D) * 2 < (1ll << 31) &&
+         (rows * a.v_ss + a.D) * 2 < (1ll << 31);
 }
 
 // Few queries per KV head (at most the 32 columns of a block) and keys enough
@@ -1318,9 +1320,7 @@ static bool flash_dec_ok(const FlashArgs& a) {
   // 32 x 32 / 8 heads 14.8 against 12).
   if (hides_past_diagonal(a) && (int64_t)a.B * a.H < 512) return false;
   return fill && (int64_t)(a.H / a.Hkv) * a.Sq <= fa::kDecCols && a.Sk >= 2 * fa::BKV &&
-         pairs < (1 << 20) && a.k_ss >= 0 && a.v_ss >= 0 &&
-         ((int64_t)a.Sk * a.k_ss + a.D) * 2 < (1ll << 31) &&
-         ((int64_t)a.Sk * a.v_ss + a.D) * 2 < (1ll << 31);
+         pairs < (1 << 20) && flash_buf_ok(a);
 }
 
 // Key tiles per split: the fewest rounds of tiles over the CUs (two waves a
