@@ -139,7 +139,7 @@ void launch_gemm(const GemmArgs& g, const StripPlan& strip, hipStream_t stream);
 // `rows` is set (a gather from the token matrix), else packed row r.  C is
 // written at its packed row.  The per-element arithmetic is the 256x256
 // kernel's (same MFMA sequence over the same k order), so a group's rows
-// equal the dense GEMM's rows bit for bit.  Fields of GemmArgs keep their
+// equal the rows of a dense GEMM that is not split bit for bit.  Fields of GemmArgs keep their
 // meaning except: a = the A matrix (token matrix when gathering) with M its
 // row count; b, b2, bias, bias2 ignored (taken from the tables); c = the
 // packed output with c_sm its row stride.
