@@ -1235,15 +1235,16 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t 
     // B's zeros are negative from the next multiple of 16 on, where the other
     // kernels' chains end: 0 * -0 leaves a sum of -0 (of products that underflow)
     // as it is, where 0 * 0 would make it +0.  (One bit-field insert in place of
-    // keep's and; z from the slot's k in the tile, which the loop does not change.)
+    // keep's and; z, whether the slot's k in the tile is 16 or more, is the same for
+    // every tile.)
     const uint32_t neg = K16 & 16 ? 0x80000000u : 0u;
-    auto keep_b = [&](float v, int k, int kin) {
-      const uint32_t m = (uint32_t)((k - K) >> 31), z = kin >= 16 ? neg : 0u;
+    auto keep_b = [&](float v, int k, uint32_t z) {
+      const uint32_t m = (uint32_t)((k - K) >> 31);
       return vm::as_f((vm::as_u(v) & m) | (z & ~m));
     };
-    auto keep4_b = [&](const float* v, int k, int kin) {
-      return make_float4(keep_b(v[0], k, kin), keep_b(v[1], k, kin), keep_b(v[2], k, kin),
-                         keep_b(v[3], k, kin));
+    auto keep4_b = [&](const float* v, int k, uint32_t z) {
+      return make_float4(keep_b(v[0], k, z), keep_b(v[1], k, z), keep_b(v[2], k, z),
+                         keep_b(v[3], k, z));
     };
     auto keep4 = [&](const float* v, int k) {
       return make_float4(keep(v[0], k), keep(v[1], k), keep(v[2], k), keep(v[3], k));
@@ -1258,17 +1259,26 @@ __global__ void __launch_bounds__(256) gemm_f32_mfma_kernel(GemmArgs g, int64_t 
         As[s][a_k ? e >> 5 : e % FM][k] = keep(ra[i], k0 + k);
       }
     }
+    // (bit 4 of the thread as a sign bit, counted anew: held in a register through
+    // the loop it takes the RW 2, ANY form past 256 of them, and half the waves)
+    uint32_t bit4 = 0;
+    if constexpr (BM == ANY) {
+      bit4 = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      asm volatile("v_lshlrev_b32 %0, 27, %0" : "+v"(bit4));
+    }
 #pragma unroll
     for (int i = 0; i < (BM == ANY ? 8 : 2); ++i) {
       const int e = tid + i * 256;
       if constexpr (BM == VEC_K) {
-        *(float4*)&Bs[s][(e >> 3) * KP + (e & 7) * 4] = keep4_b(rb + 4 * i, k0 + (e & 7) * 4, (e & 7) * 4);
+        *(float4*)&Bs[s][(e >> 3) * KP + (e & 7) * 4] =
+            keep4_b(rb + 4 * i, k0 + (e & 7) * 4, tid & 4 ? neg : 0u);
       } else if constexpr (BM == VEC_N) {
         *(float4*)&Bs[s][(e >> 4) * NP + (e & 15) * 4] =
-            keep4_b(rb + 4 * i, k0 + (e >> 4), 16 * i);
+            keep4_b(rb + 4 * i, k0 + (e >> 4), i ? neg : 0u);
       } else {
         const int k = b_k ? e & 31 : e >> 6;
-        Bs[s][k * NP + (b_k ? e >> 5 : e & 63)] = keep_b(rb[i], k0 + k, k);
+        Bs[s][k * NP + (b_k ? e >> 5 : e & 63)] =
+            keep_b(rb[i], k0 + k, (b_k ? bit4 : (uint32_t)i << 29) & neg);
       }
     }
   };
@@ -1383,15 +1393,19 @@ static F32Forms f32_forms(const GemmArgs& g) {
 // / 518, 64 x 7 x 1 363 / 535, 1 x 7 x 64 289 / 365, 33 x 7 x 33 555 / 587, 2 x
 // 33 x 2 608 / 736, 3 x 8 x 3 308 / 373; past these lines 5 x 17 x 5 584 / 593
 // and 33 x 8 x 33 570 / 475, and with 16-byte loads on both sides 8 x 8 x 8 323
-// / 231.
+// / 231.  A few hundred products are one round of either, and the lines lie
+// nearer (300 of 13 x 8 x 13 9.9 / 8.3, 7 x 5 x 7 9.8 / 9.3, 3 x 17 x 3 10.2 /
+// 9.2, but 2 x 8 x 2 7.7 / 8.3, 64 x 5 x 1 8.4 / 9.4, 1 x 17 x 1 8.8 / 9.8).
 static bool f32_generic_better(const GemmArgs& g) {
   if (g.M > kFT || g.N > kFT) return false;
   const F32Forms f = f32_forms(g);
   const int vecs = f.a_k + (f.b_k || f.b_n);
   const int64_t mn = g.M * g.N;
+  const bool many = g.batch >= 1024;
   if (vecs == 2) return false;
-  if (vecs == 1) return g.K < 8 || (g.K == 8 && mn <= 256);
-  return g.K <= 16 || (g.K <= 48 && mn <= 16);
+  if (vecs == 1) return g.K < 8 || (g.K == 8 && (mn <= 9 || (many && mn <= 256)));
+  if (g.K <= 16) return many || mn <= 16 || g.M == 1 || g.N == 1;
+  return g.K <= 48 && (mn <= 4 || (many && mn <= 16));
 }
 
 // f32 operands and result, index arithmetic that fits 32 bits, and a launch
