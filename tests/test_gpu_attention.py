@@ -136,6 +136,25 @@ def test_flash_mask_directions(gpu, oracle, direction, code, S):
     bf16_close(got, oracle.sdpa(q, k, v, code, mixed=True))
 
 
+@pytest.mark.parametrize("Sq,Sk", [(256, 256), (300, 300), (4, 200)])
+@pytest.mark.parametrize("direction", ["EQ", "NE"])
+def test_flash_unordered_masks(gpu, oracle, direction, Sq, Sk):
+    """Only the query's own key, or all but it: every tile takes the general step."""
+    B, H, Hkv, D = 1, 4, 2, 64
+    q, k, v = _qkv(oracle, 78, B, H, Hkv, Sq, Sk, D)
+
+    def fn():
+        kt, vt = E.fromHost(k, DType.BFLOAT16), E.fromHost(v, DType.BFLOAT16)
+        return _sdpa_dir(E.fromHost(q, DType.BFLOAT16), _expand(kt, B, Hkv, 2, Sk, D),
+                         _expand(vt, B, Hkv, 2, Sk, D), direction)
+
+    got, names = _run(fn)
+    assert any(n.startswith("flash_attn") for n in names), names
+    bf16_close(got, _run(fn, op_by_op=True)[0])
+    if direction == "EQ":
+        np.testing.assert_array_equal(got, np.repeat(v[:, :, :Sq], 2, axis=1))
+
+
 def test_flash_masked_keys_do_not_leak(gpu, oracle):
     """Under rew's mask query i sees keys j >= i: changing keys/values below
     the first query of the last tile leaves that tile's outputs unchanged."""
@@ -159,7 +178,8 @@ def test_flash_masked_keys_do_not_leak(gpu, oracle):
 
 
 @pytest.mark.parametrize("Sq,kernel", [(40, "flash_attn["), (1, "flash_attn_dec")])
-@pytest.mark.parametrize("Sk,D", [(129, 128), (300, 64), (191, 32), (1001, 128), (50, 64)])
+@pytest.mark.parametrize("Sk,D", [(129, 128), (300, 64), (191, 32), (1001, 128), (50, 64), (33, 32),
+                                  (1, 128)])
 def test_flash_infinite_values_over_ragged_keys(gpu, oracle, Sq, kernel, Sk, D):
     """An infinite V is an infinity in its output column, and the other columns
     keep their bits: nothing that fills up a ragged last key tile (keys seen
